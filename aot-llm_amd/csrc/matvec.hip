@@ -2172,8 +2172,185 @@ static void launch_mm_q8(const MvArgs &a, int m, hipStream_t s) {
 #undef Q8L
 }
 
-// F16 / BF16 / F32 rows (4-byte aligned rows): stage = 64 elements x 64
-// tokens of f32 input.
+// F16 / BF16 / F32 rows of whole 8-value groups on the f32 matrix cores.
+// v_mfma_f32_16x16x4_f32 is four fused multiply-adds in k order, each rounded
+// once (equal to fmaf bit for bit, denormals and infinities included), so it
+// runs four steps of one of the reference's 8 chains for 16 rows x 16 tokens:
+// chain l takes the values 8g + l of groups g = 4s..4s+3, and lane
+// (k = lane / 16, i = lane % 16) holds group 4s + k of row / token i, which is
+// 16 (F32: 32) consecutive bytes of a weight row and 32 of an input. Eight of
+// these, one per chain, take a 16x16 tile four groups on.
+// Block = 4 waves = 64 rows x 16 TT tokens, wave = 16 rows. A stage is 16
+// groups: whole-line global loads two stages ahead in registers, then LDS, two
+// stages in turn (operands straight from memory, one 16-byte piece of a row
+// per lane, 48 against 30 us at 4096x4096 and 64 tokens). A 16-byte piece
+// sits at slot 4i + (k ^ (i / 2 % 4)) of its step so that the reads of 8
+// lanes, a row stride apart, cover all banks (no bank conflicts counted).
+// Groups past the last enter as 0 and -0, whose product leaves any
+// accumulator as it is.
+// Bound by the matrix cores: a tile step is 8 x 32 clocks and a lone wave per
+// SIMD spends about 60% of its time in them. F16 4096x4096: 37 tokens 147 ->
+// 30 us, 2 tokens 234 -> 29; 14336x4096 at 64 tokens 269 -> 91 us; F32
+// 4096x4096 266 -> 38 us (against the VALU kernel below).
+typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
+typedef uint32_t u4u_t __attribute__((ext_vector_type(4), aligned(4)));
+constexpr int FX_STEP = 1024 + 64;  // bytes of 64 slots, padded: the steps of a row start 16 banks apart
+
+template <int KIND>
+__device__ __forceinline__ float fx_elem(const u32x4_t *w, int l) {
+    if (KIND == AOTK_F32) return __uint_as_float(w[l >> 2][l & 3]);
+    const uint32_t d = w[0][l >> 1];
+    if (KIND == AOTK_BF16) return __uint_as_float((l & 1) ? d & 0xFFFF0000u : d << 16);
+    return (float)__builtin_bit_cast(_Float16, (uint16_t)((l & 1) ? d >> 16 : d));
+}
+
+template <int KIND, int TT>
+__global__ __launch_bounds__(256) void k_mm_fx(MvArgs a, int m) {
+    constexpr int WP = KIND == AOTK_F32 ? 2 : 1;  // 16-byte pieces of a weight group
+    __shared__ __align__(16) uint8_t sw[2][4][4 * WP * FX_STEP];  // [stage][wave][step, piece]
+    __shared__ __align__(16) uint8_t sx[2][TT][8 * FX_STEP];      // [stage][token tile][step, piece]
+    const int tid = threadIdx.x, lane = tid & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int k = lane >> 4, i16 = lane & 15;
+    const int t0 = blockIdx.y * (16 * TT), row0 = blockIdx.x * 64;
+    const int n8 = (int)(a.cols >> 3), stages = (n8 + 15) >> 4;
+    const auto slot = [](int i, int kk) { return 16 * (4 * i + (kk ^ ((i >> 1) & 3))); };
+    // loads of a stage: each wave its 16 rows' 256 WP bytes (4 WP passes of
+    // 4 / WP rows), the block the tokens' 512 bytes (2 TT passes of 8 tokens)
+    constexpr int WL = 4 * WP, RPP = 4 / WP, LPR = 16 * WP;
+    const uint8_t *wp[WL];
+#pragma unroll
+    for (int u = 0; u < WL; u++) {
+        const int grow = min(row0 + wave * 16 + RPP * u + lane / LPR, a.total_rows - 1);
+        int local;
+        const int sg = seg_of(a, grow, local);
+        wp[u] = seg_sel(sg, a.w[0], a.w[1], a.w[2]) + (size_t)local * a.rb;
+    }
+    const int wg = (lane % LPR) / WP, wpc = (lane % LPR) % WP;  // the lane's group of the stage, its piece
+    const int xg = (tid & 31) >> 1, xpc = tid & 1;
+    const float *xp[2 * TT];
+#pragma unroll
+    for (int u = 0; u < 2 * TT; u++) xp[u] = a.xf + (size_t)min(t0 + 8 * u + (tid >> 5), m - 1) * a.cols + 4 * xpc;
+    struct Stg {
+        u32x4_t w[WL];
+        f4_t x[2 * TT];
+    };
+    auto fetch = [&](Stg &r, int st) {
+        const int gw = min(16 * st + wg, n8 - 1), gx = min(16 * st + xg, n8 - 1);
+#pragma unroll
+        for (int u = 0; u < WL; u++) r.w[u] = *(const u4u_t *)(wp[u] + (size_t)gw * (16 * WP) + 16 * wpc);
+#pragma unroll
+        for (int u = 0; u < 2 * TT; u++) r.x[u] = *(const f4u_t *)(xp[u] + (size_t)gx * 8);
+    };
+    const int full = n8 >> 4;
+    auto put = [&](Stg &r, int st, int b) {
+        if (st >= full) {  // (block-uniform) the neutral pair past the last group
+            const bool won = 16 * st + wg < n8, xon = 16 * st + xg < n8;
+#pragma unroll
+            for (int u = 0; u < WL; u++) r.w[u] = won ? r.w[u] : u32x4_t{0, 0, 0, 0};
+#pragma unroll
+            for (int u = 0; u < 2 * TT; u++) r.x[u] = xon ? r.x[u] : f4_t{-0.0f, -0.0f, -0.0f, -0.0f};
+        }
+#pragma unroll
+        for (int u = 0; u < WL; u++)
+            *(u32x4_t *)(sw[b][wave] + ((wg >> 2) * WP + wpc) * FX_STEP + slot(RPP * u + lane / LPR, wg & 3)) = r.w[u];
+#pragma unroll
+        for (int u = 0; u < 2 * TT; u++)
+            *(f4_t *)(sx[b][u >> 1] + ((xg >> 2) * 2 + xpc) * FX_STEP + slot(8 * (u & 1) + (tid >> 5), xg & 3)) = r.x[u];
+    };
+    f4_t acc[TT][8];
+#pragma unroll
+    for (int t = 0; t < TT; t++)
+#pragma unroll
+        for (int l = 0; l < 8; l++) acc[t][l] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    const int mine = slot(i16, k);
+    struct Ops {  // the operands of one step
+        u32x4_t w[WP];
+        f4_t x[TT][2];
+    };
+    auto read = [&](Ops &o, int b, int s) {
+#pragma unroll
+        for (int p = 0; p < WP; p++) o.w[p] = *(const u32x4_t *)(sw[b][wave] + (s * WP + p) * FX_STEP + mine);
+#pragma unroll
+        for (int t = 0; t < TT; t++)
+#pragma unroll
+            for (int p = 0; p < 2; p++) o.x[t][p] = *(const f4_t *)(sx[b][t] + (s * 2 + p) * FX_STEP + mine);
+    };
+    // (a change between vector and f32 matrix instructions costs a lone wave
+    // about 14 clocks and the two do not overlap: all conversions first)
+    auto step = [&](const Ops &o) {
+        float wv[8];
+#pragma unroll
+        for (int l = 0; l < 8; l++) wv[l] = fx_elem<KIND>(o.w, l);
+        __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+        for (int l = 0; l < 8; l++)
+#pragma unroll
+            for (int t = 0; t < TT; t++)
+                acc[t][l] = __builtin_amdgcn_mfma_f32_16x16x4f32(wv[l], o.x[t][l >> 2][l & 3], acc[t][l], 0, 0, 0);
+    };
+    Stg r0, r1;
+    Ops o0, o1;
+    fetch(r0, 0);
+    fetch(r1, 1);
+    put(r0, 0, 0);
+    fetch(r0, 2);
+    __syncthreads();
+    read(o0, 0, 0);
+    // Stage st is in LDS, st + 1 in `r`, st + 2 in flight. Each step's
+    // operands are read during the step before; the barrier stands before
+    // the last step, when every wave has read the stage's last operands.
+    auto stage = [&](int st, int b, Stg &r) {
+        put(r, st + 1, b ^ 1);
+        fetch(r, st + 3);
+        read(o1, b, 1);
+        __builtin_amdgcn_sched_barrier(0);
+        step(o0);
+        read(o0, b, 2);
+        __builtin_amdgcn_sched_barrier(0);
+        step(o1);
+        read(o1, b, 3);
+        __builtin_amdgcn_sched_barrier(0);
+        step(o0);
+        __syncthreads();
+        read(o0, b ^ 1, 0);
+        __builtin_amdgcn_sched_barrier(0);
+        step(o1);
+    };
+    // (an odd count ends with a stage of neutral operands)
+    for (int st = 0; st < stages; st += 2) {
+        stage(st, 0, r1);
+        stage(st + 1, 1, r0);
+    }
+    // lane (k, i): rows 4k..4k+3, token i
+#pragma unroll
+    for (int t = 0; t < TT; t++) {
+        const int tok = t0 + 16 * t + i16;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            float c[8];
+#pragma unroll
+            for (int l = 0; l < 8; l++) c[l] = acc[t][l][i];
+            const int grow = row0 + wave * 16 + 4 * k + i;
+            if (tok < m && grow < a.total_rows) store_row(a, grow, tok, hsum8(c));
+        }
+    }
+}
+
+// Two token tiles per block where that takes no more rounds of blocks over
+// the 256 CUs (fewer readers of each weight), else one. F16 14336x4096 at 64
+// tokens: 91 us with two, 99 with one; 4096x4096: 49 with two, 30 with one.
+template <int KIND>
+static void launch_mm_fx(const MvArgs &a, int m, hipStream_t s) {
+    const unsigned gx = (unsigned)((a.total_rows + 63) / 64), tiles = (unsigned)((m + 15) / 16);
+    const unsigned r1 = (gx * tiles + 255) / 256, r2 = 2 * ((gx * ((tiles + 1) / 2) + 255) / 256);
+    if (r2 <= r1) k_mm_fx<KIND, 2><<<dim3(gx, (tiles + 1) / 2), 256, 0, s>>>(a, m);
+    else k_mm_fx<KIND, 1><<<dim3(gx, tiles), 256, 0, s>>>(a, m);
+}
+
+// F16 / BF16 / F32 rows of other widths (4-byte aligned rows, a scalar tail;
+// whole 8-value groups take k_mm_fx): stage = 64 elements x 64 tokens of f32
+// input.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_mm_float(MvArgs a, int m) {
     __shared__ __align__(16) float sx[2][8][64][8];  // [stage][group of 8][token][element]
@@ -2454,6 +2631,14 @@ static void launch_args(int kind, const MvArgs &a, size_t m, hipStream_t s) {
     if (m >= MM_MIN_TOKENS && (((kind == AOTK_Q8_0 || kind == AOTK_Q4_0 || kind == AOTK_Q5_0) && a.xh) ||
                                ((kind == AOTK_F16 || kind == AOTK_BF16 || kind == AOTK_F32) && mm_float_fits(a, kind)))) {
         dim3 g((unsigned)((a.total_rows + 4 * MQ_R - 1) / (4 * MQ_R)), (unsigned)((m + 63) / 64));
+        if ((kind == AOTK_F16 || kind == AOTK_BF16 || kind == AOTK_F32) && a.cols % 8 == 0) {
+            // whole 8-value groups: the f32 matrix cores, faster at every
+            // row and token count measured (2 to 100 tokens)
+            if (kind == AOTK_F16) launch_mm_fx<AOTK_F16>(a, (int)m, s);
+            else if (kind == AOTK_BF16) launch_mm_fx<AOTK_BF16>(a, (int)m, s);
+            else launch_mm_fx<AOTK_F32>(a, (int)m, s);
+            return;
+        }
         switch (kind) {
         case AOTK_Q8_0: launch_mm_q8<AOTK_Q8_0>(a, (int)m, s); break;
         case AOTK_Q4_0: launch_mm_q8<AOTK_Q4_0>(a, (int)m, s); break;

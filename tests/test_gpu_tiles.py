@@ -1,0 +1,47 @@
+"""The batched kernels at the edges of their tiles, bit for bit against the
+CPU oracle (the reference's order of every f32 sum, so no tolerance)."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+F32, F16, BF16, Q4_0, Q5_0, Q8_0, Q4_K, Q5_K, Q6_K = range(9)
+
+
+def same_bits(got, ref):
+    return np.array_equal(np.asarray(got).view(np.uint32), np.asarray(ref).view(np.uint32))
+
+
+@pytest.mark.parametrize("kind,cols,rows,m", [
+    (F16, 8, 1, 2), (F16, 120, 63, 15), (F16, 128, 64, 16), (F16, 136, 65, 17), (F16, 2568, 130, 37), (F16, 264, 9000, 64),
+    (BF16, 24, 65, 3), (BF16, 1024, 131, 64), (BF16, 1160, 17, 100), (BF16, 256, 8200, 33),
+    (F32, 8, 17, 2), (F32, 248, 64, 31), (F32, 512, 129, 65), (F32, 136, 8256, 48)])
+def test_float_matmul_tiles(aotk, oracle, kind, cols, rows, m):
+    """Rows of whole 8-value groups: remainders of the 16-group stages (odd
+    and even stage counts), of the 64-row blocks and of one and two token
+    tiles, with exponents down to the subnormals."""
+    rng = np.random.default_rng(cols + rows + m)
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    w[:, ::7] *= np.float32(2.0 ** -18)  # f16 subnormals
+    xs = (rng.standard_normal((m, cols)) * np.exp2(rng.integers(-70, 20, (m, cols)))).astype(np.float32)
+    xs[0] = np.float32(-1e-42) * np.sign(xs[0])  # products that underflow to signed zeros
+    raw = oracle.quantize_rows(kind, w)
+    h = aotk.Weight(kind, raw, rows, cols)
+    got = aotk.matmul(h, xs, m)
+    h.free()
+    ref = oracle.matmul(kind, raw, np.ascontiguousarray(xs).view(np.uint8).reshape(-1), m, rows, cols,
+                        pool=oracle.Pool(8)).reshape(m, rows)
+    assert same_bits(got, ref)
+
+
+@pytest.mark.parametrize("kind", [F16, F32])
+def test_float_matmul_two_matrices(aotk, oracle, kind):
+    """The gate / up pair: a 64-row block over the boundary of the two."""
+    rng = np.random.default_rng(4 + kind)
+    rows, cols, m = 83, 384, 21
+    raws = [oracle.quantize_rows(kind, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)) for _ in range(2)]
+    xs = rng.standard_normal((m, cols)).astype(np.float32)
+    ws = [aotk.Weight(kind, r, rows, cols) for r in raws]
+    got = aotk.matmul2(ws[0], ws[1], xs, m)
+    for g, r in zip(got, raws):
+        assert same_bits(g, oracle.matmul(kind, r, xs.view(np.uint8).reshape(-1), m, rows, cols).reshape(m, rows))
