@@ -70,7 +70,13 @@ struct ActQ8K {
 struct ActQ8_0 {
     int8_t *qs;     // [rows][n]
     float *d;       // [rows][n/32]
-    uint16_t *xh;   // [rows][n] the quants as f16, written for batches of 2 or more (matrix-core products)
+    // Batches of 2 or more: the quants as f16 in the matrix-core operand
+    // order (null = none), 1 KB per 16-vector tile and block of 32, tiles
+    // outer: [tile][block][group q < 4][vector v % 16][groups q, q + 4 of 4
+    // values] (see k_mm_q8).
+    uint16_t *xh;
+    int tok;  // vector index of this view's first row
+    int nbt;  // blocks of 32 per vector of the tiled copy
 };
 
 // Bytes of an activation buffer for `rows` vectors of n elements.
@@ -99,8 +105,14 @@ __host__ __device__ inline size_t q8k_tiled_off(size_t v, int sb, int nbt, int e
     const int j = e >> 5, g = (e >> 3) & 3;
     return ((v >> 4) * (size_t)nbt + sb) * 4096 + (size_t)((j >> 1) * 1024 + (g * 16 + (int)(v & 15)) * 16 + (j & 1) * 8 + (e & 7));
 }
+// Value index in the tiled f16 copy of element e of block b of vector v.
+__host__ __device__ inline size_t q80_tiled_off(size_t v, int b, int nbt, int e) {
+    const int q = (e >> 2) & 3, half = e >> 4;
+    return ((v >> 4) * (size_t)nbt + b) * 512 + (size_t)((q * 16 + (int)(v & 15)) * 8 + half * 4 + (e & 3));
+}
 inline size_t act_q8_0_bytes(size_t n, size_t rows) {
-    return align_up(rows * n, 256) + align_up(rows * (n / 32) * 4, 256) + align_up(rows * n * 2, 256);
+    return align_up(rows * n, 256) + align_up(rows * (n / 32) * 4, 256) +
+           (rows >= 2 ? align_up(align_up(rows, 16) * n * 2, 256) : 0);
 }
 inline ActQ8_0 act_q8_0_view(void *base, size_t n, size_t rows) {
     uint8_t *p = (uint8_t *)base;
@@ -109,7 +121,9 @@ inline ActQ8_0 act_q8_0_view(void *base, size_t n, size_t rows) {
     p += align_up(rows * n, 256);
     a.d = (float *)p;
     p += align_up(rows * (n / 32) * 4, 256);
-    a.xh = (uint16_t *)p;
+    a.xh = rows >= 2 ? (uint16_t *)p : nullptr;
+    a.tok = 0;
+    a.nbt = (int)(n / 32);
     return a;
 }
 

@@ -1929,23 +1929,31 @@ __device__ __forceinline__ float hsum8(const float (&c)[8]) {
 
 // Q8_0 / Q4_0 / Q5_0 on the f16 matrix cores. The reference's integer part
 // per block is, for each of the 8 lanes of its accumulator, a sum of 4
-// consecutive products P_l (exact: |q| <= 127, |P_l| <= 64516). Here one
-// v_mfma_f32_16x16x32_f16 forms P for 4 rows x 16 tokens x 4 of the 8
-// groups: A holds the 4 rows' block in group-diagonal form (M index 4r + i
-// carries group 2i, or 2i + 1 in the odd product, every other entry zero),
-// B the 16 tokens' activations; the values are integers exact in f16 and
-// every partial sum is an integer below 2^24, so the f32 result is P itself.
-// Lane (q, n) then owns the 8 chains of row q and token n: the f32 fold
-// acc_l = fma(f16(d) * y.d, P_l, acc_l) over blocks in order and the avx2
-// horizontal sum run on the VALU exactly as in the matvec.
-// Wave = SETS sets of 4 rows x TILES tiles of 16 tokens; block = 4 waves
-// over BR rows x 64 tokens. The activations arrive as f16 (ActQ8_0::xh,
-// written by the batch's quantizer), the weights are converted to f16 when
-// staged; both are
-// staged in LDS, BS blocks per stage (2 or 4 by the matrix height), two
-// stages in LDS and two more in registers in flight.
-constexpr int MQ_BS = 2;   // blocks of 32 per stage
-constexpr int MQ_XS = 40;  // halves per (block, token) line of the activation tile (32 + pad)
+// consecutive products P_l (exact: |q| <= 127, |P_l| <= 64516).
+// v_mfma_f32_4x4x4_16b_f16 is sixteen independent 4x4 products of depth 4:
+// with A's blocks broadcast along the token axis (cbsz 2) and B's along the
+// row axis (blgp), one of them is P_l for 16 rows x 16 tokens, and eight take
+// a block of 32. A lane's 16 bytes of either operand are groups q and q + 4
+// of its row / token (q = lane / 4 % 4 for rows, lane / 16 for tokens), the
+// other lanes' groups reach it by the broadcast selects, so neither operand
+// is held twice. The operands are integers exact in f16 and every partial
+// sum is below 2^24: the f32 result is P_l itself. The scale products
+// f16(d) * y.d of the 16x16 outputs come from v_mfma_f32_4x4x1_f32 (one
+// rounded product per output; four blocks' scales per operand register).
+// Lane (g, n) owns the chains of rows 4g..4g+3 and token n: acc_l =
+// fma(D, P_l, acc_l) over blocks in order on the VALU, then the avx2
+// horizontal sum, as in the matvec: a batch equals m matvecs bit for bit.
+// Bound by issue: per tile and block 64 + 8 clocks of matrix products and 32
+// fma of 2.4, which barely overlap. Q8_0 at 64 tokens, against 16x16x32
+// products with the groups laid out diagonally (7 of 8 factors zero) and the
+// activations staged in LDS: 12288x4096 82 -> 50 us, 4096x12288 114 -> 62,
+// 24576x4096 120 -> 96; 5632x2048 at 6 tokens 30 -> 14 (Q5_0 32 -> 16).
+// Wave = one 16-token tile x CH of the 8 chains; block = 16 rows x 16 NT
+// tokens. The weights are converted to f16 into LDS once per block, 8 blocks
+// of 32 per stage; the activations come straight from the operand-ordered
+// copy (ActQ8_0::xh), one contiguous 1 KB per wave and block.
+constexpr int MQ_BS = 8;               // blocks of 32 per stage
+constexpr int MQ_BLK = 64 * 16 + 16;   // bytes per (stage block): 64 lanes' operands, padded against bank conflicts of the staging writes
 
 typedef _Float16 h4_t __attribute__((ext_vector_type(4)));
 typedef _Float16 h8_t __attribute__((ext_vector_type(8)));
@@ -1962,213 +1970,237 @@ __device__ __forceinline__ void u8x4_to_f16(uint32_t u, float bias, uint32_t &lo
     hi = __builtin_bit_cast(uint32_t, __builtin_bit_cast(h2_t, h) + off);
 }
 
-template <int KIND, int SETS, int TILES, int BS = MQ_BS>
-__global__ __launch_bounds__(256) void k_mm_q8(MvArgs a, int m) {
-    constexpr int WTW = 4 / TILES;      // waves along the tokens
-    constexpr int WRW = 4 / WTW;        // waves along the rows
-    constexpr int BR = WRW * 4 * SETS;  // weight rows per block
+// P of chain q (+ 4 in the upper half): the selects are immediates.
+template <int Q>
+__device__ __forceinline__ f4_t mq_chain(h4_t a, h4_t b) {
+    return __builtin_amdgcn_mfma_f32_4x4x4f16(a, b, f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 2, Q, 4 + Q);
+}
+template <int Q>
+__device__ __forceinline__ f4_t mq_scale(float a, float b) {
+    return __builtin_amdgcn_mfma_f32_4x4x1f32(a, b, f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 2, Q, 4 + Q);
+}
+
+template <int KIND, int CH, int NT>
+__global__ __launch_bounds__(64 * NT * (8 / CH), CH == 8 ? 3 : 4) void k_mm_q8(MvArgs a, int m) {
+    constexpr int NH = 8 / CH;                       // waves sharing a tile's chains
+    constexpr int T = 64 * NT * NH;                  // threads
     constexpr int QB = KIND == AOTK_Q8_0 ? 32 : 16;  // quant bytes per block
-    constexpr int WPT = KIND == AOTK_Q8_0 ? 2 : 1;   // 16-byte quant loads per (row, block)
-    constexpr int WT = BR * BS * WPT;                // weight staging loads per stage
-    constexpr int WP = (WT + 255) / 256;             // ... per thread
-    constexpr int YP = (64 * BS + 255) / 256;        // activation scales per thread
-    static_assert((BS & (BS - 1)) == 0, "stage blocks");
-    __shared__ __align__(16) _Float16 sx[2][BS][64][MQ_XS];  // activations
-    __shared__ __align__(16) float sxd[2][BS][64];           // their scales
-    __shared__ __align__(16) _Float16 sw[2][BR][BS][32];     // weight quants
-    __shared__ __align__(16) float swd[2][BR][BS];           // f32(d)
-    __shared__ __align__(16) _Float16 szero[8];
+    constexpr int WPT = KIND == AOTK_Q8_0 ? 2 : 1;   // 16-byte quant pieces per (row, block)
+    constexpr int WT = 16 * MQ_BS * WPT;             // pieces per stage
+    constexpr int WP = (WT + T - 1) / T;             // ... per thread
+    __shared__ __align__(16) uint8_t sw[2][MQ_BS * MQ_BLK];  // [stage][block][lane][halves: group q, group q + 4]
     const int tid = threadIdx.x, lane = tid & 63;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int wr = wave / WTW, wt = wave % WTW;
-    const int t0 = blockIdx.y * 64;
+    const int half = NH == 2 ? wave / NT : 0;  // chains 4 half .. of the wave (CH = 4)
     const int nb = a.nb;
-    const int row0 = blockIdx.x * BR;
-    const int mt = min(64, m - t0);
-    if (tid < 4) ((uint32_t *)szero)[tid] = 0u;
-    // the weight rows / blocks / 16-byte parts this thread stages (pass k: c = tid + 256 k)
+    const int row0 = blockIdx.x * 16;
+    const int tile = blockIdx.y * NT + wave % NT, ntiles = (m + 15) >> 4;
+    const bool active = tile < ntiles;  // (a wave past the last tile computes it again and stores nothing)
+    // the pieces this thread stages: row c / (BS WPT), block (c / WPT) % BS, part c % WPT
     const uint8_t *wq[WP];
-    const uint16_t *wd[WP];
     const uint32_t *wh[WP];
 #pragma unroll
     for (int k = 0; k < WP; k++) {
-        const int c = min(tid + 256 * k, WT - 1);
-        const int grow = min(row0 + c / (WPT * BS), a.total_rows - 1);
+        const int c = min(tid + T * k, WT - 1);
         int local;
-        const int sg = seg_of(a, grow, local);
+        const int sg = seg_of(a, min(row0 + c / (WPT * MQ_BS), a.total_rows - 1), local);
         wq[k] = seg_sel(sg, a.w[0], a.w[1], a.w[2]) + (size_t)local * nb * QB;
-        wd[k] = (const uint16_t *)seg_sel(sg, a.w1[0], a.w1[1], a.w1[2]) + (size_t)local * nb;
         wh[k] = KIND == AOTK_Q5_0 ? (const uint32_t *)seg_sel(sg, a.w2[0], a.w2[1], a.w2[2]) + (size_t)local * nb : nullptr;
     }
-    // stage loads (tokens past m and blocks past the end repeat the last:
-    // valid memory, never stored)
     struct Ld {
-        u32x4_t x[BS], w[WP];
-        float xd[YP];
-        uint32_t wd[WP], wh[WP];
+        u32x4_t w[WP];
+        uint32_t h[WP];
     };
-    Ld L[2];
-    auto fetch = [&](Ld &ld, int c0) {
-#pragma unroll
-        for (int k = 0; k < BS; k++) {  // 64 tokens x BS blocks x 4 parts of 16 bytes
-            const int c = tid + 256 * k;
-            const int t = min(t0 + c / (4 * BS), m - 1), b = min(c0 + ((c >> 2) & (BS - 1)), nb - 1);
-            ld.x[k] = *(const u32x4_t *)(a.xh + (size_t)t * a.cols + (size_t)b * 32 + (c & 3) * 8);
-        }
-#pragma unroll
-        for (int k = 0; k < YP; k++) {
-            const int c = tid + 256 * k;  // (token c / BS, block c % BS)
-            if (c < 64 * BS) {
-                const int t = min(t0 + c / BS, m - 1), b = min(c0 + (c & (BS - 1)), nb - 1);
-                ld.xd[k] = a.xd[(size_t)t * nb + b];
-            }
-        }
+    auto fetch = [&](Ld &r, int st) {  // (blocks past the end re-read the last; their scales are zero)
 #pragma unroll
         for (int k = 0; k < WP; k++) {
-            const int c = tid + 256 * k;  // (row c / (WPT BS), block (c / WPT) % BS, part c % WPT)
-            if (c < WT) {
-                const int part = c % WPT, b = min(c0 + (c / WPT) % BS, nb - 1);
-                ld.w[k] = *(const u32x4_t *)(wq[k] + (size_t)b * QB + part * 16);
-                if (KIND == AOTK_Q5_0) ld.wh[k] = wh[k][b];
-                if (part == 0) ld.wd[k] = wd[k][b];
-            }
+            const int c = tid + T * k, b = min(st * MQ_BS + (c / WPT) % MQ_BS, nb - 1);
+            r.w[k] = *(const u32x4_t *)(wq[k] + (size_t)b * QB + (c % WPT) * 16);
+            if (KIND == AOTK_Q5_0) r.h[k] = wh[k][b];
         }
     };
-    auto put = [&](const Ld &ld, int st) {
-#pragma unroll
-        for (int k = 0; k < BS; k++) {
-            const int c = tid + 256 * k;
-            *(u32x4_t *)&sx[st][(c >> 2) & (BS - 1)][c / (4 * BS)][(c & 3) * 8] = ld.x[k];
-        }
-#pragma unroll
-        for (int k = 0; k < YP; k++) {
-            const int c = tid + 256 * k;
-            if (c < 64 * BS) sxd[st][c & (BS - 1)][c / BS] = ld.xd[k];
-        }
+    auto put = [&](const Ld &r, int buf) {
 #pragma unroll
         for (int k = 0; k < WP; k++) {
-            const int c = tid + 256 * k;
-            if (c >= WT) continue;
-            const int part = c % WPT, blk = (c / WPT) % BS, row = c / (WPT * BS);
-            uint32_t *dst = (uint32_t *)&sw[st][row][blk][part * 16];
+            const int c = tid + T * k;
+            if (WT % T != 0 && c >= WT) continue;
+            const int row = c / (WPT * MQ_BS);
+            // lane (g, t, i) of row 4g + i holds groups t and t + 4
+            uint8_t *dst = sw[buf] + ((c / WPT) % MQ_BS) * MQ_BLK + (row >> 2) * 256 + (row & 3) * 16;
             if (KIND == AOTK_Q8_0) {
-                uint32_t h[8];
-#pragma unroll
-                for (int i = 0; i < 4; i++) u8x4_to_f16(ld.w[k][i] ^ 0x80808080u, 128.0f, h[2 * i], h[2 * i + 1]);
-                *(u32x4_t *)dst = u32x4_t{h[0], h[1], h[2], h[3]};
-                *(u32x4_t *)(dst + 4) = u32x4_t{h[4], h[5], h[6], h[7]};
-            } else {
-                // elements 0..15: low nibbles, 16..31: high nibbles (quant.rs:300-443)
-                uint32_t h[16];
 #pragma unroll
                 for (int i = 0; i < 4; i++) {
-                    uint32_t l4 = ld.w[k][i] & 0x0F0F0F0Fu, h4 = (ld.w[k][i] >> 4) & 0x0F0F0F0Fu;
+                    uint2 h;
+                    u8x4_to_f16(r.w[k][i] ^ 0x80808080u, 128.0f, h.x, h.y);
+                    *(uint2 *)(dst + 64 * i + 8 * (c % WPT)) = h;
+                }
+            } else {
+                // elements 0..15: low nibbles, 16..31: high nibbles (quant.rs:300-443)
+#pragma unroll
+                for (int i = 0; i < 4; i++) {
+                    uint32_t l4 = r.w[k][i] & 0x0F0F0F0Fu, h4 = (r.w[k][i] >> 4) & 0x0F0F0F0Fu;
                     if (KIND == AOTK_Q5_0) {
-                        const uint32_t bl = (ld.wh[k] >> (4 * i)) & 0xFu, bh = (ld.wh[k] >> (16 + 4 * i)) & 0xFu;
+                        const uint32_t bl = (r.h[k] >> (4 * i)) & 0xFu, bh = (r.h[k] >> (16 + 4 * i)) & 0xFu;
                         l4 |= ((bl & 1u) | ((bl & 2u) << 7) | ((bl & 4u) << 14) | ((bl & 8u) << 21)) << 4;
                         h4 |= ((bh & 1u) | ((bh & 2u) << 7) | ((bh & 4u) << 14) | ((bh & 8u) << 21)) << 4;
                     }
                     const float bias = KIND == AOTK_Q5_0 ? 16.0f : 8.0f;
-                    u8x4_to_f16(l4, bias, h[2 * i], h[2 * i + 1]);
-                    u8x4_to_f16(h4, bias, h[8 + 2 * i], h[8 + 2 * i + 1]);
-                }
-#pragma unroll
-                for (int i = 0; i < 4; i++) *(u32x4_t *)(dst + 4 * i) = u32x4_t{h[4 * i], h[4 * i + 1], h[4 * i + 2], h[4 * i + 3]};
-            }
-            if (part == 0) swd[st][row][blk] = f16_to_f32(ld.wd[k]);
-        }
-    };
-    // lane roles: q = lane / 16 (the output row in a set of 4, and the
-    // operands' k-quarter), n = lane % 16 (the token in a tile; as an A row
-    // index, row n / 4 of the set with group pair n % 4)
-    const int q = lane >> 4, n = lane & 15;
-    const bool a_on = (n & 3) == q;  // A[4r + i][k] is nonzero only in k-quarter i
-    const int a_row = n >> 2;
-    f4_t acc[SETS][TILES][2];  // [row set][token tile][even / odd groups]
-#pragma unroll
-    for (int s = 0; s < SETS; s++)
-#pragma unroll
-        for (int t = 0; t < TILES; t++) acc[s][t][0] = acc[s][t][1] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
-    fetch(L[0], 0);
-    if (BS < nb) fetch(L[1], BS);
-    put(L[0], 0);
-    __syncthreads();
-    // one stage: stage c0 + 2 * BS goes into the register set `fr` just
-    // emptied, the stage in `pr` (fetched a round earlier) into the other
-    // LDS buffer after the compute (last read in the previous round, before
-    // its barrier)
-    auto round = [&](int c0, int st, Ld &fr, const Ld &pr) {
-        if (c0 + 2 * BS < nb) fetch(fr, c0 + 2 * BS);
-        const int nblk = nb - c0 < BS ? nb - c0 : BS;
-        for (int j = 0; j < nblk; j++) {
-            h8_t bx[TILES];
-            float yd[TILES];
-#pragma unroll
-            for (int t = 0; t < TILES; t++) {
-                const int tok = 16 * (wt * TILES + t) + n;
-                bx[t] = *(const h8_t *)&sx[st][j][tok][8 * q];
-                yd[t] = sxd[st][j][tok];
-            }
-#pragma unroll
-            for (int s = 0; s < SETS; s++) {
-                const int r0 = 4 * (wr * SETS + s);  // first row of the set in the block
-                const _Float16 *ap = a_on ? &sw[st][r0 + a_row][j][8 * q] : szero;
-                const h4_t lo = *(const h4_t *)ap, hi = *(const h4_t *)(ap + 4);
-                const _Float16 z = (_Float16)0;
-                const h8_t ae = {lo[0], lo[1], lo[2], lo[3], z, z, z, z};
-                const h8_t ao = {z, z, z, z, hi[0], hi[1], hi[2], hi[3]};
-                const float dw = swd[st][r0 + q][j];
-#pragma unroll
-                for (int t = 0; t < TILES; t++) {  // (tiles past the batch compute on repeated tokens)
-                    const f4_t pe = __builtin_amdgcn_mfma_f32_16x16x32_f16(ae, bx[t], f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    const f4_t po = __builtin_amdgcn_mfma_f32_16x16x32_f16(ao, bx[t], f4_t{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
-                    const float D = dw * yd[t];
-#pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        acc[s][t][0][i] = fmaf(D, pe[i], acc[s][t][0][i]);
-                        acc[s][t][1][i] = fmaf(D, po[i], acc[s][t][1][i]);
-                    }
+                    uint4 h;
+                    u8x4_to_f16(l4, bias, h.x, h.y);
+                    u8x4_to_f16(h4, bias, h.z, h.w);
+                    *(uint4 *)(dst + 64 * i) = h;
                 }
             }
         }
-        if (c0 + BS < nb) {
-            put(pr, st ^ 1);
-            __syncthreads();
-        }
     };
-    for (int c0 = 0; c0 < nb; c0 += 2 * BS) {
-        round(c0, 0, L[0], L[1]);
-        if (c0 + BS < nb) round(c0 + BS, 1, L[1], L[0]);
+    // operands of a quarter stage (4 blocks): the tokens' quants, and one
+    // scale per lane: block 4s + t of row 4g + i in lane (g, t, i), block
+    // 4s + q of token n in lane (q, n)
+    const int g = lane >> 4, t4 = (lane >> 2) & 3, n = lane & 15;
+    const uint16_t *dw;
+    {
+        int local;
+        const int sg = seg_of(a, min(row0 + 4 * g + (lane & 3), a.total_rows - 1), local);
+        dw = (const uint16_t *)seg_sel(sg, a.w1[0], a.w1[1], a.w1[2]) + (size_t)local * nb;
     }
-    // lane (q, n): row r0 + q of each set, token 16 * tile + n; groups 2i (even) and 2i + 1 (odd)
+    const float *dx = a.xd + (size_t)min(tile * 16 + n, m - 1) * nb;
+    const uint8_t *xt = (const uint8_t *)a.xh + (size_t)min(tile, ntiles - 1) * nb * 1024 + lane * 16 + (NH == 2 ? 8 * half : 0);
+    struct Op {
+        u32x4_t x[4];  // (CH = 4: the low 8 bytes)
+        uint32_t dw;
+        float dx;
+    };
+    auto load = [&](Op &o, int s) {
 #pragma unroll
-    for (int s = 0; s < SETS; s++) {
-        const int grow = row0 + 4 * (wr * SETS + s) + q;
-#pragma unroll
-        for (int t = 0; t < TILES; t++) {
-            const int tt = 16 * (wt * TILES + t) + n;
-            const f4_t e = acc[s][t][0], o = acc[s][t][1];
-            // ((a0+a4)+(a2+a6)) + ((a1+a5)+(a3+a7))  (simd_avx2.rs:27-34), a_{2i} = e[i], a_{2i+1} = o[i]
-            const float v = ((e[0] + e[2]) + (e[1] + e[3])) + ((o[0] + o[2]) + (o[1] + o[3]));
-            if (tt < mt && grow < a.total_rows) store_row(a, grow, t0 + tt, v);
+        for (int t = 0; t < 4; t++) {
+            const uint8_t *p = xt + (size_t)min(4 * s + t, nb - 1) * 1024;
+            if (CH == 8) o.x[t] = *(const u32x4_t *)p;
+            else {
+                const uint2 v = *(const uint2 *)p;
+                o.x[t][0] = v.x;
+                o.x[t][1] = v.y;
+            }
         }
+        const int bw = 4 * s + t4, bx = 4 * s + g;
+        o.dw = dw[min(bw, nb - 1)];
+        o.dx = dx[min(bx, nb - 1)];
+    };
+    f4_t acc[CH];
+#pragma unroll
+    for (int l = 0; l < CH; l++) acc[l] = f4_t{0.0f, 0.0f, 0.0f, 0.0f};
+    auto fold = [&](f4_t &c, const f4_t &D, const f4_t &P) {
+#pragma unroll
+        for (int i = 0; i < 4; i++) c[i] = fmaf(D[i], P[i], c[i]);
+    };
+    auto compute = [&](const Op &o, int s, int buf) {
+        // (masks, not selects: no branch, so that the waits for the loads in flight stay exact)
+        const float da = __uint_as_float(__float_as_uint(f16_to_f32(o.dw)) & (uint32_t)((4 * s + t4 - nb) >> 31));
+        const float db = __uint_as_float(__float_as_uint(o.dx) & (uint32_t)((4 * s + g - nb) >> 31));
+        const f4_t D[4] = {mq_scale<0>(da, db), mq_scale<1>(da, db), mq_scale<2>(da, db), mq_scale<3>(da, db)};
+        typedef _Float16 wop_t __attribute__((ext_vector_type(CH)));
+        wop_t w[4];  // (all four blocks' reads before the first use)
+#pragma unroll
+        for (int t = 0; t < 4; t++)
+            w[t] = *(const wop_t *)(sw[buf] + ((4 * s + t) & (MQ_BS - 1)) * MQ_BLK + lane * 16 + (NH == 2 ? 8 * half : 0));
+#pragma unroll
+        for (int t = 0; t < 4; t++) {
+            h4_t wl = {w[t][0], w[t][1], w[t][2], w[t][3]}, wu, xl, xu;
+            if (CH == 8) {
+                const h8_t x = __builtin_bit_cast(h8_t, o.x[t]);
+                wu = h4_t{w[t][CH - 4], w[t][CH - 3], w[t][CH - 2], w[t][CH - 1]};
+                xl = h4_t{x[0], x[1], x[2], x[3]}, xu = h4_t{x[4], x[5], x[6], x[7]};
+            } else {
+                xl = __builtin_bit_cast(h4_t, uint2{o.x[t][0], o.x[t][1]});
+            }
+            f4_t P[CH];
+            P[0] = mq_chain<0>(wl, xl);
+            P[1] = mq_chain<1>(wl, xl);
+            P[2] = mq_chain<2>(wl, xl);
+            P[3] = mq_chain<3>(wl, xl);
+            if (CH == 8) {
+                P[CH - 4] = mq_chain<0>(wu, xu);
+                P[CH - 3] = mq_chain<1>(wu, xu);
+                P[CH - 2] = mq_chain<2>(wu, xu);
+                P[CH - 1] = mq_chain<3>(wu, xu);
+            }
+#pragma unroll
+            for (int l = 0; l < CH; l++) {
+                fold(acc[l], D[t], P[l]);
+                asm volatile("" : "+v"(acc[l]));  // (here, not sunk past the block: P would stay in registers)
+            }
+        }
+    };
+    const int stages = (nb + MQ_BS - 1) / MQ_BS;
+    Ld r0, r1;
+    constexpr int NO = CH == 8 ? 2 : 4;  // quarter stages in flight per wave
+    Op o[NO];
+    fetch(r0, 0);
+    fetch(r1, 1);
+#pragma unroll
+    for (int k = 0; k < NO; k++) load(o[k], k);
+    put(r0, 0);
+    __syncthreads();
+    auto stage = [&](int st, int buf, Ld &next, Ld &after, Op &oa, Op &ob) {
+        put(next, buf ^ 1);
+        fetch(after, st + 2);
+        compute(oa, 2 * st, buf);
+        load(oa, 2 * st + NO);
+        compute(ob, 2 * st + 1, buf);
+        load(ob, 2 * st + 1 + NO);
+        __syncthreads();
+    };
+    // (an odd stage count ends with a stage of zero scales)
+    for (int st = 0; st < stages; st += 2) {
+        stage(st, 0, r1, r0, o[0], o[1]);
+        stage(st + 1, 1, r0, r1, o[NO - 2], o[NO - 1]);
+    }
+    // ((a0+a4)+(a2+a6)) + ((a1+a5)+(a3+a7))  (simd_avx2.rs:27-34)
+    if (NH == 2) {  // the upper chains meet the lower ones in LDS
+        f4_t *up = (f4_t *)sw + (wave % NT) * 256 + lane;
+        if (half == 1)
+#pragma unroll
+            for (int l = 0; l < 4; l++) up[64 * l] = acc[l];
+        __syncthreads();
+        if (half == 1 || !active) return;
+        const int tok = tile * 16 + n;
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            const float c[8] = {acc[0][i], acc[1][i], acc[2][i], acc[3][i], up[0][i], up[64][i], up[128][i], up[192][i]};
+            if (tok < m && row0 + 4 * g + i < a.total_rows) store_row(a, row0 + 4 * g + i, tok, hsum8(c));
+        }
+        return;
+    }
+    if (!active) return;
+    const int tok = tile * 16 + n;
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+        float c[8];
+#pragma unroll
+        for (int l = 0; l < 8; l++) c[l] = acc[l % CH][i];
+        if (tok < m && row0 + 4 * g + i < a.total_rows) store_row(a, row0 + 4 * g + i, tok, hsum8(c));
     }
 }
 
 template <int KIND>
 static void launch_mm_q8(const MvArgs &a, int m, hipStream_t s) {
-    // (the quants as f16 come with the batch: written by its quantizer)
-    // rows per block by the matrix height: enough waves for few rows, more
-    // reuse of each staged activation for many
-    const unsigned gy = (unsigned)((m + 63) / 64);
-    // (sets, tiles, blocks per stage) measured at 64 tokens: 4096 rows
-    // (1, 2, 4) against (2, 1, 2) 46 / 59 us at 4096 columns, 126 / 164 us
-    // at 12288; 6144 rows (2, 2, 4) 63 against 72 us; 24576 rows (2, 4, 2)
-    // 137 against 142 us for 4 blocks per stage
-#define Q8L(S, T, B) k_mm_q8<KIND, S, T, B><<<dim3((unsigned)((a.total_rows + 4 * S * T - 1) / (4 * S * T)), gy), 256, 0, s>>>(a, m)
-    if (a.total_rows >= 16384) Q8L(2, 4, 2);
-    else if (a.total_rows >= 6144) Q8L(2, 2, 4);
-    else Q8L(1, 2, 4);
+    const unsigned gx = (unsigned)((a.total_rows + 15) / 16);
+    const int tiles = (m + 15) / 16;
+    const int gy = (tiles + 3) / 4, nt = (tiles + gy - 1) / gy;
+    const dim3 grid(gx, (unsigned)gy);
+    // A tile's chains on two waves for at most 32 tokens a block, where the
+    // SIMDs would otherwise hold too few waves (Q8_0, 16 tokens: 4096x4096 20
+    // against 26 us, 12288x4096 31 against 35, 4096x12288 59 against 73); on
+    // one wave above (64 tokens: 24 against 26, 50 against 76, 62 against 77:
+    // two waves form every scale product and read every operand line twice).
+    const bool split = nt <= 2;
+#define Q8L(C, N) k_mm_q8<KIND, C, N><<<grid, 64 * N * (8 / C), 0, s>>>(a, m)
+    if (split) {
+        if (nt == 1) Q8L(4, 1);
+        else Q8L(4, 2);
+    } else {
+        if (nt == 3) Q8L(8, 3);
+        else Q8L(8, 4);
+    }
 #undef Q8L
 }
 

@@ -132,7 +132,8 @@ __device__ __forceinline__ ActQ8_0 q80_row(ActQ8_0 a, size_t row, size_t n) {
     ActQ8_0 r = a;
     r.qs += row * n;
     r.d += row * (n / 32);
-    if (r.xh) r.xh += row * n;
+    r.tok = (int)row;
+    r.nbt = (int)(n / 32);
     return r;
 }
 

@@ -45,3 +45,34 @@ def test_float_matmul_two_matrices(aotk, oracle, kind):
     got = aotk.matmul2(ws[0], ws[1], xs, m)
     for g, r in zip(got, raws):
         assert same_bits(g, oracle.matmul(kind, r, xs.view(np.uint8).reshape(-1), m, rows, cols).reshape(m, rows))
+
+
+@pytest.mark.parametrize("kind", [Q8_0, Q4_0, Q5_0])
+@pytest.mark.parametrize("cols,rows,m", [
+    (32, 1, 2), (96, 17, 15), (256, 16, 16), (288, 33, 17), (480, 47, 32), (512, 48, 33), (544, 15, 48),
+    (2048, 131, 49), (2080, 64, 64), (352, 20, 65), (736, 49, 100), (1024, 9, 130)])
+def test_q80_family_matmul_tiles(aotk, oracle, kind, cols, rows, m):
+    """Remainders of the 4- and 8-block stages (odd and even stage counts),
+    the 16-row blocks, and one to four token tiles on one or two waves each."""
+    rng = np.random.default_rng(cols + rows + m + kind)
+    raw = oracle.quantize_rows(kind, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    xs = (rng.standard_normal((m, cols)) * np.exp2(rng.integers(-6, 6, (m, 1)))).astype(np.float32)
+    acts = np.concatenate([oracle.quantize_act(kind, x) for x in xs])
+    h = aotk.Weight(kind, raw, rows, cols)
+    got = aotk.matmul(h, acts, m)
+    h.free()
+    ref = oracle.matmul(kind, raw, acts, m, rows, cols, pool=oracle.Pool(8)).reshape(m, rows)
+    assert same_bits(got, ref)
+
+
+def test_noalloc_without_room_for_the_tiled_copy(aotk, oracle):
+    """Two inputs of 204800 columns: the staging that fits the fixed memory
+    except for the copy's whole 16-vector tiles."""
+    kind, cols, rows, m = Q8_0, 204800, 3, 2
+    rng = np.random.default_rng(12)
+    raw = oracle.quantize_rows(kind, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    acts = np.concatenate([oracle.quantize_act(kind, rng.standard_normal(cols).astype(np.float32)) for _ in range(m)])
+    h = aotk.Weight(kind, raw, rows, cols)
+    got = aotk.matmul_noalloc(h, acts, m)
+    h.free()
+    assert same_bits(got, oracle.matmul(kind, raw, acts, m, rows, cols).reshape(m, rows))
