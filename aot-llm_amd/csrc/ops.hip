@@ -9,6 +9,8 @@
 // sequential order (a different order changes results by an ulp, which flips
 // int8 roundings downstream); transcendental functions are the host-libm
 // matched aotk_expf / aotk_tanhf. Maxima and integer sums use trees.
+#include <algorithm>
+
 #include "device.hpp"
 #include "lds_chain.hpp"
 #include "formats.hpp"
@@ -464,172 +466,90 @@ __global__ __launch_bounds__(512) void k_attn_scores(AttnArgs a) {
     a.prob[(i * a.n_head + (size_t)(kvh * gqa + hg)) * a.span + (start + lane - t0)] = s * a.scale;
 }
 
-// Prompt scores for ATT_SRB rows per block: block = (kv head, chunk of
-// ATT_CH absolute positions, group of ATT_SRB rows), gqa * 64 threads. The
-// chunk's K rows are staged once for the group; thread (query head,
-// position) runs the rows' dot products side by side, each sequentially over
-// the head dimension, and writes those of the rows whose range [t0, n) holds
-// the position.
-constexpr int ATT_SRB = 4;
-template <int HD>
-__global__ __launch_bounds__(512) void k_attn_scores_rb(AttnArgs a, int m) {
-    constexpr int KS = HD + 4;  // 16-byte rows; lanes reading 16 bytes of 16 rows hit all banks
-    __shared__ __align__(16) float sk[ATT_CH * KS];
-    __shared__ __align__(16) float sq[ATT_SRB][ATT_MAX_GQA][HD];
-    const int gqa = a.n_head / a.n_kv_head;
-    const int lane = threadIdx.x & 63, hg = threadIdx.x >> 6;
-    const int kvh = blockIdx.x;
-    const size_t start = (size_t)blockIdx.y * ATT_CH;
-    const int i0 = blockIdx.z * ATT_SRB;
-    size_t t0[ATT_SRB], tn[ATT_SRB];
-    size_t lo = ~(size_t)0, hi = 0;
-#pragma unroll
-    for (int r = 0; r < ATT_SRB; r++) {
-        row_range(a, (size_t)min(i0 + r, m - 1), t0[r], tn[r]);
-        if (i0 + r >= m) tn[r] = t0[r];  // rows past m: empty
-        lo = min(lo, t0[r]);
-        hi = max(hi, tn[r]);
-    }
-    if (start >= hi || start + ATT_CH <= lo) return;  // no row has a position here
-    const size_t end = min(start + ATT_CH, hi);
-    const int rows = (int)(end - start);
-    const size_t kv = (size_t)a.n_kv_head * HD, q_dim = (size_t)a.n_head * HD;
-    const int nthreads = gqa * 64;
-    for (int e = threadIdx.x; e < ATT_SRB * gqa * HD; e += nthreads) {
-        const int r = e / (gqa * HD), hh = (e / HD) % gqa, d = e % HD;
-        const size_t i = (size_t)min(i0 + r, m - 1);
-        sq[r][hh][d] = a.q[i * q_dim + (size_t)(kvh * gqa + hh) * HD + d];
-    }
-    const float *kb = a.k_cache + start * kv + (size_t)kvh * HD;
-    constexpr int R4 = HD / 4;
-    for (int idx = threadIdx.x; idx < rows * R4; idx += nthreads) {
-        const int r = idx / R4, c4 = idx % R4;
-        *(float4 *)(sk + r * KS + 4 * c4) = *(const float4 *)(kb + (size_t)r * kv + 4 * c4);
-    }
-    __syncthreads();
-    if (lane >= rows) return;
-    const size_t t = start + lane;
-    const float4 *kr = (const float4 *)(sk + lane * KS);
-    float sc[ATT_SRB];
-#pragma unroll
-    for (int r = 0; r < ATT_SRB; r++) sc[r] = 0.0f;
-#pragma unroll 2
-    for (int d4 = 0; d4 < HD / 4; d4++) {
-        const float4 k4 = kr[d4];
-#pragma unroll
-        for (int r = 0; r < ATT_SRB; r++) {
-            const float4 q4 = ((const float4 *)sq[r][hg])[d4];
-            sc[r] += q4.x * k4.x;
-            sc[r] += q4.y * k4.y;
-            sc[r] += q4.z * k4.z;
-            sc[r] += q4.w * k4.w;
-        }
-    }
-#pragma unroll
-    for (int r = 0; r < ATT_SRB; r++)
-        if (t >= t0[r] && t < tn[r])
-            a.prob[((size_t)(i0 + r) * a.n_head + (size_t)(kvh * gqa + hg)) * a.span + (t - t0[r])] = sc[r] * a.scale;
+// Products of 16 steps for four rows at once: v_mfma_f32_4x4x1_f32 with a
+// zero accumulator is one rounded product per output, x[row i] of step K
+// (held by lane 4K + i of the register `x`, broadcast to every lane's block)
+// times the lane's y[K]. Matrix and vector f32 take the same time per
+// product, but the row operand needs no register copy per lane: a broadcast
+// from LDS costs LDS bandwidth, and a DPP or scalar operand halves the
+// multiply's rate (4.6 against 2.5 clocks). A sum started at +0 is never -0,
+// so that the product's zero may lose its sign.
+typedef float att_f4 __attribute__((ext_vector_type(4)));
+template <int K = 0>
+__device__ __forceinline__ void att_prod16(att_f4 (&p)[16], float x, const float (&y)[16]) {
+    p[K] = __builtin_amdgcn_mfma_f32_4x4x1f32(x, y[K], att_f4{0.0f, 0.0f, 0.0f, 0.0f}, 4, K, 0);
+    if constexpr (K + 1 < 16) att_prod16<K + 1>(p, x, y);
 }
 
-// Wave-uniform operands through the scalar unit: loads through a pointer in
-// the constant address space become s_load (the data is not written during
-// the kernel), so a value every lane needs costs no vector load or LDS read.
-typedef const float __attribute__((address_space(4))) *att_cfp;
-typedef float att_f8 __attribute__((ext_vector_type(8)));
-__device__ __forceinline__ att_f8 att_sload8(const float *p) { return *(const __attribute__((address_space(4))) att_f8 *)p; }
-
-
-// Prompt scores: block = (kv head, chunk of 64 absolute positions, group of
-// R rows), GQA waves; thread (query head hg = wave, position = lane) runs the
-// R rows' dot products side by side, each sequentially over the head
-// dimension (s += q[d] * k[d], ops.rs:160-166), then scales them. The q
-// values are wave-uniform: scalar loads, 8 dimensions of the R rows at a
-// time. The chunk's K rows are staged in LDS 32 dimensions at a time (one
-// 16-byte read per lane and 4 dimensions), the next 32 in flight.
-constexpr int ATT_KD = 32;  // dimensions per K stage
-template <int HD, int GQA, int R>
-__global__ __launch_bounds__(64 * GQA) void k_attn_scores_sg(AttnArgs a, int m) {
-    constexpr int KS = ATT_KD + 4;
-    constexpr int NT = 64 * GQA;
-    constexpr int NL = 64 * ATT_KD / 4 / NT;  // float4 loads per thread and stage
-    static_assert(NL >= 1, "stage");
-    __shared__ __align__(16) float sk[2][64][KS];
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int hg = __builtin_amdgcn_readfirstlane(tid >> 6);
-    const int kvh = blockIdx.x;
-    const size_t start = (size_t)blockIdx.y * 64;
-    const int i0 = blockIdx.z * R;
-    size_t t0[R], tn[R];
-    size_t lo = ~(size_t)0, hi = 0;
-#pragma unroll
-    for (int r = 0; r < R; r++) {
-        row_range(a, (size_t)min(i0 + r, m - 1), t0[r], tn[r]);
-        if (i0 + r >= m) tn[r] = t0[r];  // rows past m: empty
-        lo = min(lo, t0[r]);
-        hi = max(hi, tn[r]);
-    }
-    if (start >= hi || start + 64 <= lo) return;  // no row has a position here
+// Prompt scores: block = (kv head, chunk of 64 absolute positions, row
+// group), wave = (query head, 4 RQ rows), lane = position. The chunk's K rows
+// are staged in LDS once for the block (128 dimensions at a time); a lane
+// reads its own row 16 bytes at a time and runs the rows' dot products side
+// by side, each in dimension order: products by att_prod16, one add per
+// (row, position, dimension) on the VALU, which bounds it (with q broadcast
+// from LDS the reads did: 100 us at 64 rows x 32 heads x 4032 positions,
+// head_dim 128).
+template <int HD, int RQ>
+__global__ __launch_bounds__(512) void k_attn_scores_rows(AttnArgs a, int m, int rgs) {
+    constexpr int DC = HD < 128 ? HD : 128, KS = DC + 4, R = 4 * RQ;
+    __shared__ __align__(16) float sk[ATT_CH * KS];
+    const int gqa = a.n_head / a.n_kv_head;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int kvh = blockIdx.x, h = kvh * gqa + wave % gqa;
+    const size_t start = (size_t)blockIdx.y * ATT_CH;
+    const int b0 = blockIdx.z * R * rgs, i0 = b0 + wave / gqa * R;
+    // (rows' ranges move forward with the row)
+    size_t lo, hi, tmp;
+    row_range(a, (size_t)b0, lo, tmp);
+    row_range(a, (size_t)min(b0 + R * rgs, m) - 1, tmp, hi);
+    if (start >= hi || start + ATT_CH <= lo) return;  // no row has a position here
     const size_t kv = (size_t)a.n_kv_head * HD, q_dim = (size_t)a.n_head * HD;
-    const float *qr[R];
-#pragma unroll
-    for (int r = 0; r < R; r++) qr[r] = a.q + (size_t)min(i0 + r, m - 1) * q_dim + (size_t)(kvh * GQA + hg) * HD;
-    // stage loads: position c / (ATT_KD / 4), dims 4 (c % (ATT_KD / 4)) of the stage (positions past the
-    // union's end re-read its last one)
     const float *kb = a.k_cache + (size_t)kvh * HD;
-    float4 lk[NL];
-    auto fetch = [&](int dc) {
+    const float *qp[RQ];  // lane 4b + i: dimension b of row i
 #pragma unroll
-        for (int k = 0; k < NL; k++) {
-            const int c = tid + NT * k;
-            const size_t t = min(start + (size_t)(c / (ATT_KD / 4)), hi - 1);
-            lk[k] = *(const float4 *)(kb + t * kv + dc + 4 * (c % (ATT_KD / 4)));
+    for (int r = 0; r < RQ; r++) qp[r] = a.q + (size_t)min(i0 + 4 * r + (lane & 3), m - 1) * q_dim + (size_t)h * HD + (lane >> 2);
+    float q[RQ][HD / 16];
+#pragma unroll
+    for (int r = 0; r < RQ; r++)
+#pragma unroll
+        for (int g = 0; g < HD / 16; g++) q[r][g] = qp[r][16 * g];
+    float s[RQ][4];
+#pragma unroll
+    for (int r = 0; r < RQ; r++) s[r][0] = s[r][1] = s[r][2] = s[r][3] = 0.0f;
+#pragma unroll
+    for (int c = 0; c < HD; c += DC) {
+        if (c) __syncthreads();
+        for (int idx = threadIdx.x; idx < ATT_CH * (DC / 4); idx += blockDim.x) {
+            const int r = idx / (DC / 4), c4 = idx % (DC / 4);
+            *(float4 *)(sk + r * KS + 4 * c4) = *(const float4 *)(kb + min(start + r, hi - 1) * kv + c + 4 * c4);
         }
-    };
-    auto put = [&](int buf) {
+        __syncthreads();
 #pragma unroll
-        for (int k = 0; k < NL; k++) {
-            const int c = tid + NT * k;
-            *(float4 *)&sk[buf][c / (ATT_KD / 4)][4 * (c % (ATT_KD / 4))] = lk[k];
-        }
-    };
-    fetch(0);
-    put(0);
-    __syncthreads();
-    float sc[R];
+        for (int g = 0; g < DC / 16; g++) {
+            float k[16];
 #pragma unroll
-    for (int r = 0; r < R; r++) sc[r] = 0.0f;
-    int buf = 0;
-    for (int dc = 0; dc < HD; dc += ATT_KD) {
-        const bool more = dc + ATT_KD < HD;
-        if (more) fetch(dc + ATT_KD);
+            for (int j = 0; j < 4; j++) *(float4 *)&k[4 * j] = *(const float4 *)(sk + lane * KS + 16 * g + 4 * j);
 #pragma unroll
-        for (int d8 = 0; d8 < ATT_KD; d8 += 8) {
-            att_f8 q8[R];
+            for (int r = 0; r < RQ; r++) {
+                att_f4 p[16];
+                att_prod16(p, q[r][c / 16 + g], k);
 #pragma unroll
-            for (int r = 0; r < R; r++) q8[r] = att_sload8(qr[r] + dc + d8);
+                for (int d = 0; d < 16; d++)
 #pragma unroll
-            for (int h = 0; h < 2; h++) {
-                const float4 k4 = *(const float4 *)&sk[buf][lane][d8 + 4 * h];
+                    for (int i = 0; i < 4; i++) s[r][i] += p[d][i];
 #pragma unroll
-                for (int r = 0; r < R; r++) {
-                    sc[r] = sc[r] + q8[r][4 * h] * k4.x;
-                    sc[r] = sc[r] + q8[r][4 * h + 1] * k4.y;
-                    sc[r] = sc[r] + q8[r][4 * h + 2] * k4.z;
-                    sc[r] = sc[r] + q8[r][4 * h + 3] * k4.w;
-                }
+                for (int i = 0; i < 4; i++) asm volatile("" : "+v"(s[r][i]));  // (the adds here: sunk, the products would stay in registers)
             }
-        }
-        if (more) {
-            put(buf ^ 1);  // the other buffer was last read before the previous barrier
-            __syncthreads();
-            buf ^= 1;
         }
     }
     const size_t t = start + lane;
 #pragma unroll
-    for (int r = 0; r < R; r++)
-        if (t >= t0[r] && t < tn[r])
-            a.prob[((size_t)(i0 + r) * a.n_head + (size_t)(kvh * GQA + hg)) * a.span + (t - t0[r])] = sc[r] * a.scale;
+    for (int r = 0; r < R; r++) {
+        if (i0 + r >= m) break;
+        size_t t0, n;
+        row_range(a, (size_t)(i0 + r), t0, n);
+        if (t >= t0 && t < n) a.prob[((size_t)(i0 + r) * a.n_head + h) * a.span + (t - t0)] = s[r / 4][r % 4] * a.scale;
+    }
 }
 
 // One wave's share of the q/k/v epilogue for one head vector (decode):
@@ -1160,178 +1080,126 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_decode1(AttnArgs a, QkvPost p) {
 }
 
 // Batched rows (prompt chunks), spans up to ATT_MAX_SPAN: the same softmax
-// and output, with the serial chains spread over lanes instead of blocks.
-//   k_attn_softmax_rows: one wave per (row, head) for spans up to
-//   ATT_ROWS_MAX: max, glibc-matched exp into LDS, the sequential sum by
-//   lane 0, then p = e * (1 / sum) written back over the scores; longer
-//   spans: k_attn_softmax_rows_x, a block per (row, head).
-//   k_attn_out_rows: one wave per (head, 64-dim slice, ATT_RB rows: 2 at
-//   head_dim <= 128, 1 at 256); lane d keeps the ATT_RB sums of dim d and
-//   adds p_t * v_t,d in position order;
-//   V rows are read straight from the cache (256 B per wave per position),
-//   the probabilities with wave-uniform loads.
-constexpr int ATT_ROWS_MAX = 2048;  // spans of the one-wave softmax (four waves per block)
+// and output, with the serial chains spread over lanes instead of blocks:
+// k_attn_softmax_rows_p / _x, then k_attn_out_rows.
 
-template <int NW, int CAP>
-__global__ __launch_bounds__(64 * NW) void k_attn_softmax_rows(AttnArgs a, int m) {
-    __shared__ __align__(16) float e[NW][CAP];
-    __shared__ uint64_t stab[32];  // expf's 2^(i/32) table (an LDS read per lookup)
-    const int lane = threadIdx.x & 63, w = threadIdx.x >> 6;
-    const int pair = blockIdx.x * NW + w;
-    exp_table_to_lds(stab);
-    __syncthreads();
-    if (pair >= m * a.n_head) return;
-    const int i = pair / a.n_head, h = pair % a.n_head;
-    size_t t0, n;
-    row_range(a, i, t0, n);
-    const int cnt = (int)(n - t0);
-    float *ps = a.prob + ((size_t)i * a.n_head + h) * a.span;
-    float *ew = e[w];
-    // every score load of the lane in flight together (a loop that stores
-    // each one as it arrives waits for the loads one at a time)
-    constexpr int VPL = CAP / 64;
-    float v[VPL];
-    float mx = -INFINITY;
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int t = lane + 64 * k;
-        v[k] = t < cnt ? ps[t] : -INFINITY;
-    }
-#pragma unroll
-    for (int k = 0; k < VPL; k++) mx = fmaxf(mx, v[k]);
-    mx = wave_max(mx);
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int t = lane + 64 * k;
-        if (t < cnt) {
-            v[k] = aotk_expf_tab(v[k] - mx, stab);
-            ew[t] = v[k];
-        }
-    }
-    if (cnt + lane < ((cnt + 63) & ~63)) ew[cnt + lane] = -0.0f;  // neutral padding to a run of 64
-    wave_lds_sync();
-    float sum = 0.0f;
-    if (lane == 0) sum = seq_sum_lds_pad64(ew, cnt);
-    const float inv = 1.0f / readlane_f(sum, 0);
-#pragma unroll
-    for (int k = 0; k < VPL; k++) {
-        const int t = lane + 64 * k;
-        if (t < cnt) ps[t] = v[k] * inv;
-    }
-}
-
-template <int HD, int ATT_RB, int GS = 32>
-__global__ __launch_bounds__(256) void k_attn_out_rows(AttnArgs a, int m) {
-    static_assert(ATT_RB == 4 || ATT_RB == 2 || ATT_RB == 1, "one float4 / float2 / float of p per position");
-    static_assert((GS == 32 || GS == 64) && GS * ATT_RB <= 128, "positions per group: the p slot holds 128 floats");
-    __shared__ float4 sPr[4][32];
+// Prompt output: wave = (kv head, 64 dimensions, NI consecutive items of
+// (token, query head of the group)), lane = dimension: the lane's NI sums run
+// over the positions in order, products by att_prod16 (lane 4K + i holds item
+// i's probability of position K of each 16), one add per (item, position) on
+// the VALU. V and the probabilities come straight from memory, 64 positions
+// ahead in registers; the waves of a block (consecutive items of one kv head
+// and slice) share V's lines in the L1. A wave alone on its SIMD issues an
+// instruction per 4.7 clocks, which bounds it: 16 products and 16 NI adds per
+// 16 positions, kept apart (a change between matrix and vector f32 costs 14).
+template <int HD, int NI>
+__global__ __launch_bounds__(256, 1) void k_attn_out_rows(AttnArgs a, int m) {
     constexpr int NS = HD / 64;
-    const int lane = threadIdx.x & 63;
-    const int wv = threadIdx.x >> 6;
-    const int task = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);  // wave-uniform
-    const int slice = task % NS, h = (task / NS) % a.n_head, rg = task / (NS * a.n_head);
-    if (rg * ATT_RB >= m) return;
-    const int gqa = a.n_head / a.n_kv_head, kvh = h / gqa;
+    const int gqa = a.n_head / a.n_kv_head;
+    const int lane = threadIdx.x & 63, wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int slice = blockIdx.x % NS, kvh = (blockIdx.x / NS) % a.n_kv_head;
+    const int items = m * gqa, it0 = (blockIdx.x / (NS * a.n_kv_head) * 4 + wave) * NI;
+    if (it0 >= items) return;
     const size_t kv = (size_t)a.n_kv_head * HD;
-    const int d = slice * 64 + lane;
-    int row[ATT_RB];
-    size_t t0[ATT_RB], tn[ATT_RB];
-    const float *pr[ATT_RB];
-    size_t lo = ~(size_t)0, hi = 0, alo = 0, ahi = ~(size_t)0;
+    // the items' ranges (items past the last repeat it, unstored), from the first one's start
+    size_t lo, tmp;
+    row_range(a, (size_t)(it0 / gqa), lo, tmp);
+    int t0[NI], tn[NI];
 #pragma unroll
-    for (int r = 0; r < ATT_RB; r++) {
-        row[r] = min(rg * ATT_RB + r, m - 1);  // rows past m repeat the last one, unstored
-        row_range(a, row[r], t0[r], tn[r]);
-        pr[r] = a.prob + ((size_t)row[r] * a.n_head + h) * a.span - t0[r];
-        lo = min(lo, t0[r]);
-        hi = max(hi, tn[r]);
-        alo = max(alo, t0[r]);
-        ahi = min(ahi, tn[r]);
+    for (int i = 0; i < NI; i++) {
+        size_t x, y;
+        row_range(a, (size_t)(min(it0 + i, items - 1) / gqa), x, y);
+        t0[i] = (int)(x - lo);
+        tn[i] = (int)(y - lo);
     }
-    const float *vb = a.v_cache + (size_t)kvh * HD + d;
-    float o[ATT_RB];
+    const int alo = t0[NI - 1], ahi = tn[0], cnt = tn[NI - 1];  // common to all: [alo, ahi)
+    // groups of 16 positions that all items hold: [gs, ge)
+    const int gs = (alo + 15) >> 4, ge = max(gs, ahi >> 4);
+    // this lane's probability operand: item lane % 4, position lane / 4 of each 16
+    const int mine = min(it0 + min(lane & 3, NI - 1), items - 1), mt = mine / gqa;
+    const float *pr = a.prob + ((size_t)mt * a.n_head + (size_t)kvh * gqa + mine % gqa) * a.span;
+    size_t mx, my;
+    row_range(a, (size_t)mt, mx, my);
+    const int m0 = (int)(mx - lo), m1 = (int)(my - lo);
+    const float *vb = a.v_cache + lo * kv + (size_t)kvh * HD + slice * 64;  // (wave-uniform)
+    float o[NI];
 #pragma unroll
-    for (int r = 0; r < ATT_RB; r++) o[r] = 0.0f;
-    auto step_if = [&](size_t t) {
-        const float v = vb[t * kv];
+    for (int i = 0; i < NI; i++) o[i] = 0.0f;
+    auto load_p = [&](int t) { return pr[max(min(t + (lane >> 2), m1 - 1), m0) - m0]; };
+    // a group that some item does not hold whole, or past the end
+    auto edge = [&](int g) {
+        const int t = 16 * g;
+        float y[16];
+        att_f4 x[16];
 #pragma unroll
-        for (int r = 0; r < ATT_RB; r++)
-            if (t >= t0[r] && t < tn[r]) o[r] += pr[r][t] * v;
+        for (int k = 0; k < 16; k++) y[k] = vb[(size_t)min(t + k, cnt - 1) * kv + lane];
+        att_prod16(x, load_p(t), y);
+#pragma unroll
+        for (int k = 0; k < 16; k++)
+#pragma unroll
+            for (int i = 0; i < NI; i++)
+                if (t + k >= t0[i] && t + k < tn[i]) o[i] += x[k][i];
     };
-    if (alo >= ahi) {  // no position common to all rows
-        for (size_t t = lo; t < hi; t++) step_if(t);
-    } else {
-        for (size_t t = lo; t < alo; t++) step_if(t);
-        // groups of 32 positions in two register sets (A, B), each loaded one
-        // group ahead of its use: V with one load per position, p with one
-        // load per row (lane k holds position k), written to this wave's LDS
-        // slot as [position][row] so that one broadcast 16-byte read gives
-        // the four rows' p of a position
-        size_t t = alo;
-        float va[GS], pa[ATT_RB], vbb[GS], pb[ATT_RB];
-        float4 *sp = sPr[wv];
-        auto load = [&](float (&v)[GS], float (&pv)[ATT_RB], size_t c) {
+    for (int g = 0; g < gs; g++) edge(g);
+    if (gs < ge) {
+        constexpr int PD = 4;  // groups in flight
+        float v[PD][16], p[PD];
+        uint32_t off[16];  // a group's rows from its first: one base per group, no address arithmetic per load
 #pragma unroll
-            for (int k = 0; k < GS; k++) v[k] = vb[(c + k) * kv];
+        for (int k = 0; k < 16; k++) off[k] = (uint32_t)((size_t)k * kv) + lane;
+        auto load = [&](float (&vv)[16], float &pp, int g) {  // (groups past the last re-read it: never used)
+            const int t = 16 * min(g, ge - 1);
+            const float *base = vb + (size_t)t * kv;
 #pragma unroll
-            for (int r = 0; r < ATT_RB; r++) pv[r] = pr[r][c + (lane & (GS - 1))];
+            for (int k = 0; k < 16; k++) vv[k] = base[off[k]];
+            pp = load_p(t);
         };
-        auto use = [&](const float (&v)[GS], const float (&pv)[ATT_RB]) {
-            if (ATT_RB == 4) {
-                if (lane < GS) sp[lane] = make_float4(pv[0], pv[ATT_RB > 1 ? 1 : 0], pv[ATT_RB > 2 ? 2 : 0], pv[ATT_RB > 3 ? 3 : 0]);
-            } else if (ATT_RB == 2) {
-                if (lane < GS) ((float2 *)sp)[lane] = make_float2(pv[0], pv[ATT_RB > 1 ? 1 : 0]);
-            } else {
-                if (lane < GS) ((float *)sp)[lane] = pv[0];
-            }
-            wave_lds_sync();
+        auto add = [&](const att_f4 (&x)[16]) {
 #pragma unroll
-            for (int k = 0; k < GS; k++) {
-                if (ATT_RB == 4) {
-                    const float4 p4 = sp[k];
-                    o[0] += p4.x * v[k];
-                    o[ATT_RB > 1 ? 1 : 0] += p4.y * v[k];
-                    o[ATT_RB > 2 ? 2 : 0] += p4.z * v[k];
-                    o[ATT_RB > 3 ? 3 : 0] += p4.w * v[k];
-                } else if (ATT_RB == 2) {
-                    const float2 p2 = ((const float2 *)sp)[k];
-                    o[0] += p2.x * v[k];
-                    o[ATT_RB > 1 ? 1 : 0] += p2.y * v[k];
-                } else {
-                    o[0] += ((const float *)sp)[k] * v[k];
-                }
-            }
-            wave_lds_sync();
+            for (int k = 0; k < 16; k++)
+#pragma unroll
+                for (int i = 0; i < NI; i++) o[i] += x[k][i];
+#pragma unroll
+            for (int i = 0; i < NI; i++) asm volatile("" : "+v"(o[i]));
+            __builtin_amdgcn_sched_barrier(0);
         };
-        if (t + GS <= ahi) load(va, pa, t);
-        while (t + GS <= ahi) {
-            const bool more = t + 2 * GS <= ahi;
-            if (more) load(vbb, pb, t + GS);
-            use(va, pa);
-            t += GS;
-            if (!more) break;
-            const bool more2 = t + 2 * GS <= ahi;
-            if (more2) load(va, pa, t + GS);
-            use(vbb, pb);
-            t += GS;
-            if (!more2) break;
-        }
-        for (; t < ahi; t++) {
-            const float v = vb[t * kv];
 #pragma unroll
-            for (int r = 0; r < ATT_RB; r++) o[r] += pr[r][t] * v;
+        for (int k = 0; k < PD; k++) load(v[k], p[k], gs + k);
+        __builtin_amdgcn_sched_barrier(0);
+        // the products of a group are formed before the sums of the one before it
+        att_f4 x0[16], x1[16];
+        att_prod16(x0, p[0], v[0]);
+        load(v[0], p[0], gs + PD);
+        __builtin_amdgcn_sched_barrier(0);
+        int g = gs;
+        for (; g + PD <= ge; g += PD) {
+#pragma unroll
+            for (int k = 0; k < PD; k++) {
+                att_prod16(k & 1 ? x0 : x1, p[(k + 1) % PD], v[(k + 1) % PD]);
+                load(v[(k + 1) % PD], p[(k + 1) % PD], g + k + 1 + PD);
+                __builtin_amdgcn_sched_barrier(0);
+                add(k & 1 ? x1 : x0);
+            }
         }
-        for (t = ahi; t < hi; t++) step_if(t);
+#pragma unroll
+        for (int k = 0; k < PD - 1; k++) {
+            if (g + k < ge) {
+                att_prod16(k & 1 ? x0 : x1, p[(k + 1) % PD], v[(k + 1) % PD]);
+                add(k & 1 ? x1 : x0);
+            }
+        }
     }
+    for (int g = ge; 16 * g < cnt; g++) edge(g);
 #pragma unroll
-    for (int r = 0; r < ATT_RB; r++)
-        if (rg * ATT_RB + r < m) a.out[(size_t)row[r] * a.n_head * HD + (size_t)h * HD + d] = o[r];
+    for (int i = 0; i < NI; i++) {
+        const int it = it0 + i;
+        if (it < items) a.out[(size_t)(it / gqa) * a.n_head * HD + (size_t)(kvh * gqa + it % gqa) * HD + slice * 64 + lane] = o[i];
+    }
 }
 
-// The same for rows of more than ATT_ROWS_MAX positions: a block of SEQ_T
-// threads per (row, head), the scores held in registers through the max,
-// the exps with the 2^(i/32) table in LDS, the exact parallel replay of the
-// sequential sum (one wave's single-thread sum of 4096 terms took ~100 us).
+// Softmax of few long rows: a block of SEQ_T threads per (row, head), the
+// scores held in registers through the max, the exps with the 2^(i/32) table
+// in LDS, the exact parallel replay of the sequential sum.
 template <int CAP>
 __global__ __launch_bounds__(SEQ_T) void k_attn_softmax_rows_x(AttnArgs a, int m) {
     __shared__ __align__(16) float e[CAP + SEQ_T + 32];
@@ -1376,88 +1244,118 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_softmax_rows_x(AttnArgs a, int m
     }
 }
 
-// The same on 256 threads per (row, head) (spans up to CAP <= 8192): the
-// prompt runs m x n_head of these at once, so the issue count of the exact
-// sum matters more than its latency.
-template <int CAP>
-__global__ __launch_bounds__(256) void k_attn_softmax_rows_q(AttnArgs a, int m) {
-    constexpr int T = 256;
-    __shared__ __align__(16) float e[CAP + T + 32];
-    __shared__ SeqScratch S;
-    __shared__ float red[T / 64];
+// Softmax of prompt rows: P (row, head) pairs per block of T threads, each on
+// T / P of them with its scores in registers: max, glibc-matched exp into
+// LDS, the P sequential sums side by side, one per lane of wave 0 (rows 16
+// bytes apart in the banks), then p = e * (1 / sum) over the scores. The
+// chain's latency (about 7 clocks per position) bounds it: paid once per
+// block, and hidden by the loads and exps of other blocks only where several
+// fit a CU.
+template <int P, int CAP, int T>
+__global__ __launch_bounds__(T) void k_attn_softmax_rows_p(AttnArgs a, int m) {
+    constexpr int TP = T / P, NV = CAP / TP / 4, NW = TP / 64, RS = CAP + 4;
+    __shared__ __align__(16) float e[P * RS];
+    __shared__ float red[T / 64], sinv[P];
     __shared__ uint64_t stab[32];
-    constexpr int SPT = CAP / T;
-    const int tid = threadIdx.x, lane = tid & 63;
-    const int i = blockIdx.x / a.n_head, h = blockIdx.x % a.n_head;
-    size_t t0, n;
-    row_range(a, i, t0, n);
+    const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
+    const int r = tid / TP, u = tid % TP;
+    const int pairs = m * a.n_head, pair = min((int)blockIdx.x * P + r, pairs - 1);  // pairs past the last repeat it, unstored
+    const bool own = (int)blockIdx.x * P + r < pairs;
+    size_t t0, n, n_last;
+    row_range(a, (size_t)(pair / a.n_head), t0, n);
     const int cnt = (int)(n - t0);
-    float *ps = a.prob + ((size_t)i * a.n_head + h) * a.span;
+    // the block's longest row, in whole runs of 64 (ranges grow with the row)
+    row_range(a, (size_t)(min((int)blockIdx.x * P + P - 1, pairs - 1) / a.n_head), t0, n_last);
+    const int run = ((int)(n_last - t0) + 63) & ~63;
+    float4 *ps = (float4 *)(a.prob + (size_t)pair * a.span);
     exp_table_to_lds(stab);
-    float sv[SPT];
+    float4 v[NV];
     float mx = -INFINITY;
 #pragma unroll
-    for (int k = 0; k < SPT; k++) {
-        const int t = tid + k * T;
-        sv[k] = t < cnt ? ps[t] : -INFINITY;
-        mx = fmaxf(mx, sv[k]);
+    for (int k = 0; k < NV; k++) {
+        const int t = 4 * (u + TP * k);
+        v[k] = t < cnt ? ps[u + TP * k] : make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);  // (rows are whole float4s)
+        if (t + 1 >= cnt) v[k].y = -INFINITY;
+        if (t + 2 >= cnt) v[k].z = -INFINITY;
+        if (t + 3 >= cnt) v[k].w = -INFINITY;
     }
-    mx = wave_max(mx);
-    if (lane == 0) red[tid >> 6] = mx;
-    __syncthreads();
-    mx = wave_max(lane < T / 64 ? red[lane] : -INFINITY);
-    const int C = seq_chunk_of(cnt, T);
 #pragma unroll
-    for (int k = 0; k < SPT; k++) {
-        const int t = tid + k * T;
-        if (t < cnt) {
-            sv[k] = aotk_expf_tab(sv[k] - mx, stab);
-            e[seq_idx(t, C)] = sv[k];
+    for (int k = 0; k < NV; k++) mx = fmaxf(mx, fmaxf(fmaxf(v[k].x, v[k].y), fmaxf(v[k].z, v[k].w)));
+    mx = wave_max(mx);
+    if (lane == 0) red[w] = mx;
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < NW; k++) mx = fmaxf(mx, red[r * NW + k]);
+#pragma unroll
+    for (int k = 0; k < NV; k++) {
+        const int t = 4 * (u + TP * k);
+        if (t < run) {
+            // -0 past the row's end: neutral in the sum
+            v[k].x = t < cnt ? aotk_expf_tab(v[k].x - mx, stab) : -0.0f;
+            v[k].y = t + 1 < cnt ? aotk_expf_tab(v[k].y - mx, stab) : -0.0f;
+            v[k].z = t + 2 < cnt ? aotk_expf_tab(v[k].z - mx, stab) : -0.0f;
+            v[k].w = t + 3 < cnt ? aotk_expf_tab(v[k].w - mx, stab) : -0.0f;
+            *(float4 *)&e[r * RS + t] = v[k];
         }
     }
     __syncthreads();
-    const float inv = 1.0f / exact_seq_sum256(e, cnt, S);
+    if (tid < P) sinv[tid] = 1.0f / seq_sum_lds_pad64(e + tid * RS, run);
+    __syncthreads();
+    const float inv = sinv[r];
+    if (!own) return;
 #pragma unroll
-    for (int k = 0; k < SPT; k++) {
-        const int t = tid + k * T;
-        if (t < cnt) ps[t] = sv[k] * inv;
+    for (int k = 0; k < NV; k++) {
+        const int t = 4 * (u + TP * k);
+        if (t < cnt) ps[u + TP * k] = make_float4(v[k].x * inv, v[k].y * inv, v[k].z * inv, v[k].w * inv);
     }
 }
 
-
 static void launch_rows(const AttnArgs &a, size_t head_dim, size_t m, size_t longest, hipStream_t s) {
     const unsigned pairs = (unsigned)(m * a.n_head);
-    // many (row, head) pairs: the 256-thread exact sum for spans past 1024
-    // (measured at 64 rows x 32 heads: 4096 positions 64 -> 51 us); few
-    // pairs (8 heads at 8192 positions: 27 against 34 us) keep the
-    // 1024-thread form
-    const bool many = pairs >= 1024;
-    if (many && longest > 1024 && longest <= 4096) k_attn_softmax_rows_q<4096><<<pairs, 256, 0, s>>>(a, (int)m);
-    else if (many && longest > 4096 && longest <= 8192) k_attn_softmax_rows_q<8192><<<pairs, 256, 0, s>>>(a, (int)m);
-    else if (longest <= (size_t)ATT_ROWS_MAX) k_attn_softmax_rows<4, ATT_ROWS_MAX><<<(pairs + 3) / 4, 256, 0, s>>>(a, (int)m);
-    else if (longest <= 8192) k_attn_softmax_rows_x<8192><<<pairs, SEQ_T, 0, s>>>(a, (int)m);
-    else k_attn_softmax_rows_x<ATT_MAX_SPAN><<<pairs, SEQ_T, 0, s>>>(a, (int)m);
-    // rows per wave (measured at 64 rows against 4: head_dim 128 two rows,
-    // 4096 positions 160 -> 127 us, 512 positions 25 -> 21 us; head_dim 256
-    // one row, 8192 positions 297 -> 213 us, a 1024 window 47 -> 30 us)
-    const int RB = head_dim == 256 ? 1 : 2;
-    // V loads 64 positions ahead instead of 32 for long spans (measured:
-    // Qwen3 4096 positions 126 -> 118 us, Gemma-3 8192 206 -> 194 us,
-    // a 1024 window 29 -> 28 us; 512 positions 21 -> 23 us)
-    const bool deep = longest >= 1024;
-    const size_t tasks = (m + RB - 1) / RB * a.n_head * (head_dim / 64);
-    const unsigned g = (unsigned)((tasks + 3) / 4);
-    switch (head_dim) {
-    case 64: k_attn_out_rows<64, 2><<<g, 256, 0, s>>>(a, (int)m); break;
-    case 128:
-        if (deep) k_attn_out_rows<128, 2, 64><<<g, 256, 0, s>>>(a, (int)m);
-        else k_attn_out_rows<128, 2><<<g, 256, 0, s>>>(a, (int)m);
-        break;
-    default:
-        if (deep) k_attn_out_rows<256, 1, 64><<<g, 256, 0, s>>>(a, (int)m);
-        else k_attn_out_rows<256, 1><<<g, 256, 0, s>>>(a, (int)m);
-        break;
+#define SML(P, CAP, T) k_attn_softmax_rows_p<P, CAP, T><<<(pairs + P - 1) / P, T, 0, s>>>(a, (int)m)
+    if (pairs >= 1024 && longest <= 8192) {
+        // enough pairs for eight per block on every CU. 64 rows x 32 heads
+        // against one pair per wave, and past 1024 positions per 256 threads
+        // with the parallel replay: 512 positions 9.5 -> 7.3 us, 4096 50 ->
+        // 41; 6064 (four per block) 95 -> 78
+        if (longest <= 512) SML(8, 512, 1024);
+        else if (longest <= 1024) SML(8, 1024, 1024);
+        else if (longest <= 2048) SML(8, 2048, 1024);
+        else if (longest <= 4096) SML(8, 4096, 1024);
+        else SML(4, 8192, 1024);
+    } else if (longest <= 2048) {
+        // few pairs: more threads each (50 rows x 8 heads, a 1024 window
+        // 17.4 -> 8.0 us; 6 rows x 32 heads, 2006 positions 35 -> 12.6)
+        if (longest <= 512) SML(4, 512, 512);
+        else if (longest <= 1024) SML(2, 1024, 512);
+        else SML(2, 2048, 1024);
+    } else if (longest <= 8192) {
+        // few long rows: the parallel replay (20 rows x 8 heads, 3020
+        // positions: 8.2 us against 15 for one chain per block)
+        k_attn_softmax_rows_x<8192><<<pairs, SEQ_T, 0, s>>>(a, (int)m);
+    } else {
+        k_attn_softmax_rows_x<ATT_MAX_SPAN><<<pairs, SEQ_T, 0, s>>>(a, (int)m);
     }
+#undef SML
+    // Items per wave: as many waves as there are SIMDs first, then more items
+    // per product (each product instruction serves up to four). 64 rows x 32
+    // heads x 4032 positions (4096 / NI waves): NI 4 82 us, 2 118, 1 204
+    // (114 before, with V per wave from L2 and p from LDS); 64 rows x 8 heads
+    // x 7000, head_dim 256: NI 2 117, 4 132, 1 173 (156); 6 rows x 32 heads x
+    // 2000: NI 1 26, 2 33, 4 37 (41).
+    const size_t items = m * (a.n_head / a.n_kv_head), per = a.n_kv_head * (head_dim / 64);
+    const int NI = items * per <= 1024 ? 1 : items * per <= 2048 ? 2 : 4;
+    const unsigned g = (unsigned)(per * ((items + 4 * NI - 1) / (4 * NI)));
+#define OUTL(H)                                                              \
+    do {                                                                     \
+        if (NI == 1) k_attn_out_rows<H, 1><<<g, 256, 0, s>>>(a, (int)m);     \
+        else if (NI == 2) k_attn_out_rows<H, 2><<<g, 256, 0, s>>>(a, (int)m); \
+        else k_attn_out_rows<H, 4><<<g, 256, 0, s>>>(a, (int)m);             \
+    } while (0)
+    if (head_dim == 64) OUTL(64);
+    else if (head_dim == 128) OUTL(128);
+    else OUTL(256);
+#undef OUTL
 }
 
 static void launch_sv(const AttnArgs &a, size_t head_dim, size_t m, hipStream_t s) {
@@ -1503,28 +1401,28 @@ void launch_attention(float *out, const float *q, const float *k_cache, const fl
     size_t span = window > 0 && window < ctx_rows ? window : ctx_rows;
     dim3 grid((unsigned)n_kv_head, (unsigned)((span + ATT_CH - 1) / ATT_CH), (unsigned)m);
     const unsigned threads = (unsigned)(64 * (n_head / n_kv_head));
-    const size_t gqa_ratio = n_head / n_kv_head;
-    if (m > 1 && !pos_dev && head_dim == 256 &&
-        (gqa_ratio == 1 || gqa_ratio == 2 || gqa_ratio == 4 || gqa_ratio == 8)) {
-        // head_dim 256: rows batched per block, q through the scalar unit
-        // (measured at 64 rows: 8192 positions 839 -> 188 us, a 1024 window
-        // 68 -> 43 us; at head_dim 128 the per-row-group kernel below stays
-        // ahead, 107 against 114 us at 4096 positions)
-        const size_t hi = pos0 + m;  // the last row's end
-        const int gqa = (int)(n_head / n_kv_head);
-        dim3 g4((unsigned)n_kv_head, (unsigned)((hi + 63) / 64), (unsigned)((m + 3) / 4));
-        switch (gqa) {
-        case 1: k_attn_scores_sg<256, 1, 4><<<g4, 64, 0, s>>>(a, (int)m); break;
-        case 2: k_attn_scores_sg<256, 2, 4><<<g4, 128, 0, s>>>(a, (int)m); break;
-        case 4: k_attn_scores_sg<256, 4, 4><<<g4, 256, 0, s>>>(a, (int)m); break;
-        case 8: k_attn_scores_sg<256, 8, 4><<<g4, 512, 0, s>>>(a, (int)m); break;
-        }
-    } else if (m > 1 && !pos_dev && head_dim <= 128) {
-        // several rows per block over absolute position chunks
-        const size_t hi = pos0 + m;  // the last row's end
-        dim3 g((unsigned)n_kv_head, (unsigned)((hi + ATT_CH - 1) / ATT_CH), (unsigned)((m + ATT_SRB - 1) / ATT_SRB));
-        if (head_dim == 64) k_attn_scores_rb<64><<<g, threads, 0, s>>>(a, (int)m);
-        else k_attn_scores_rb<128><<<g, threads, 0, s>>>(a, (int)m);
+    if (m > 1 && !pos_dev) {
+        // Eight rows per wave where that still leaves about four blocks per
+        // CU, else four. 64 rows: 32 heads x 4032 positions, head_dim 128, 61
+        // us with eight, 66 with four (100 before); 8 heads x 7000, head_dim
+        // 256, 59 / 66 (146); 32 heads x 448 14.5 / 13.9 (18); 8 heads, a
+        // 1024 window, head_dim 256, 20.7 / 19.5 (37); 6 rows x 32 heads x
+        // 2000 10.5 / 8.7 (11.4).
+        const size_t held = window > 0 && window < pos0 + m ? window + m : pos0 + m;  // positions of any row
+        const int gqa = (int)(n_head / n_kv_head), rgs = std::max(1, 4 / gqa);
+        const size_t blocks8 = n_kv_head * ((held + ATT_CH - 1) / ATT_CH) * ((m + 8 * rgs - 1) / (8 * rgs));
+        const int R = blocks8 >= 1024 ? 8 : 4;
+        const dim3 g((unsigned)n_kv_head, (unsigned)((pos0 + m + ATT_CH - 1) / ATT_CH), (unsigned)((m + R * rgs - 1) / (R * rgs)));
+        const unsigned th = (unsigned)(64 * gqa * rgs);
+#define SCL(H)                                                              \
+    do {                                                                    \
+        if (R == 4) k_attn_scores_rows<H, 1><<<g, th, 0, s>>>(a, (int)m, rgs); \
+        else k_attn_scores_rows<H, 2><<<g, th, 0, s>>>(a, (int)m, rgs);      \
+    } while (0)
+        if (head_dim == 64) SCL(64);
+        else if (head_dim == 128) SCL(128);
+        else SCL(256);
+#undef SCL
     } else {
         switch (head_dim) {
         case 64: k_attn_scores<64><<<grid, threads, 0, s>>>(a); break;

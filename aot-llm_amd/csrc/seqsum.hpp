@@ -333,18 +333,6 @@ __device__ __forceinline__ float exact_seq_sum_t(const float *pp, int n, SeqScra
     return S.result;
 }
 
-// The same sum on a block of 256 threads (n <= 8192; the inputs in the
-// layout of seq_idx with C = seq_chunk_of(n, 256)): about twice the latency
-// of the 1024-thread form, half its instructions, for kernels that run many
-// independent sums at once.
-__device__ __forceinline__ float exact_seq_sum256(const float *pp, int n, SeqScratch &S) {
-    const int C = seq_chunk_of(n, 256);
-    if (C <= 4) return exact_seq_sum_t<4, 256>(pp, n, S);
-    if (C <= 8) return exact_seq_sum_t<8, 256>(pp, n, S);
-    if (C <= 16) return exact_seq_sum_t<16, 256>(pp, n, S);
-    return exact_seq_sum_t<32, 256>(pp, n, S);
-}
-
 __device__ __forceinline__ float exact_seq_sum(const float *pp, int n, SeqScratch &S) {
     if (seq_threads(n) == 256) return exact_seq_sum_t<4, 256>(pp, n, S);
     if (seq_chunk(n) <= 4) return exact_seq_sum_t<4, SEQ_T>(pp, n, S);

@@ -76,3 +76,55 @@ def test_noalloc_without_room_for_the_tiled_copy(aotk, oracle):
     got = aotk.matmul_noalloc(h, acts, m)
     h.free()
     assert same_bits(got, oracle.matmul(kind, raw, acts, m, rows, cols).reshape(m, rows))
+
+
+def attention_ref(oracle, q, kc, vc, nh, nkv, hd, ctx, pos0, m, window):
+    ref = np.zeros(m * nh * hd, np.float32)
+    p = oracle.Pool(8)
+    oracle.load().or_attention(p.p, oracle.ptr(ref), oracle.ptr(q), oracle.ptr(kc), oracle.ptr(vc), nh, nkv, hd, ctx, 0,
+                               pos0, m, window)
+    return ref
+
+
+@pytest.mark.parametrize("nh,nkv,hd,pos0,m,window", [
+    # one, two and four items per wave; groups of 16 positions cut at either
+    # end; every ratio of query to kv heads
+    (4, 4, 64, 0, 2, 0), (4, 4, 64, 14, 3, 0), (32, 4, 64, 0, 6, 0), (32, 4, 64, 505, 64, 0), (6, 2, 64, 31, 33, 20),
+    (32, 8, 128, 0, 64, 0), (32, 8, 128, 447, 64, 0), (10, 2, 128, 100, 17, 0), (12, 2, 128, 63, 40, 50),
+    (14, 2, 128, 5, 30, 0), (16, 2, 128, 130, 64, 100), (32, 8, 128, 985, 39, 0), (32, 8, 128, 1500, 33, 1024),
+    (8, 4, 256, 200, 64, 1024), (8, 4, 256, 3001, 50, 1024), (8, 4, 256, 1000, 40, 1024), (4, 4, 256, 70, 5, 64),
+    # the softmax's classes: many pairs at 512, 1024, 2048, 4096, 8192
+    # positions, few pairs likewise, past 8192
+    (32, 8, 128, 448, 64, 0), (32, 8, 128, 449, 64, 0), (32, 4, 64, 960, 64, 0), (32, 4, 64, 961, 64, 0),
+    (32, 4, 64, 1984, 64, 0), (32, 4, 64, 1985, 64, 0), (32, 4, 64, 4032, 64, 0), (32, 4, 64, 4033, 64, 0),
+    (32, 4, 64, 8128, 64, 0), (32, 4, 64, 8129, 64, 0),
+    (8, 4, 64, 508, 4, 0), (8, 4, 64, 509, 4, 0), (8, 4, 64, 1020, 4, 0), (8, 4, 64, 1021, 4, 0),
+    (8, 4, 64, 2044, 4, 0), (8, 4, 64, 2045, 4, 0), (8, 4, 64, 8188, 4, 0), (8, 4, 64, 8189, 4, 0)])
+def test_prompt_attention_tiles(aotk, oracle, nh, nkv, hd, pos0, m, window):
+    rng = np.random.default_rng(nh * 7 + hd + pos0 + m)
+    ctx = pos0 + m + 3
+    q = (rng.standard_normal(m * nh * hd) * 2).astype(np.float32)
+    kc, vc = (rng.standard_normal(ctx * nkv * hd).astype(np.float32) for _ in range(2))
+    vc[::5] *= np.float32(1e-39)  # products in the subnormals
+    got = aotk.attention(q, kc, vc, nh, nkv, hd, ctx, 0, pos0, m, window)
+    assert same_bits(got, attention_ref(oracle, q, kc, vc, nh, nkv, hd, ctx, pos0, m, window))
+
+
+@pytest.mark.parametrize("nh,nkv,hd,pos0,m,window", [(8, 4, 128, 200, 9, 0), (32, 8, 128, 70, 64, 40), (8, 4, 256, 90, 21, 32)])
+def test_prompt_attention_masks_positions(aotk, oracle, nh, nkv, hd, pos0, m, window):
+    """Infinities and NaN in cache rows that a query row does not hold (later
+    positions, positions before its window) leave it untouched."""
+    rng = np.random.default_rng(3 + pos0)
+    ctx = pos0 + m + 3
+    q = rng.standard_normal(m * nh * hd).astype(np.float32)
+    kc, vc = (rng.standard_normal((ctx, nkv * hd)).astype(np.float32) for _ in range(2))
+    want = attention_ref(oracle, q, kc.reshape(-1), vc.reshape(-1), nh, nkv, hd, ctx, pos0, m, window)
+    clean = [i for i in range(m - 2)]
+    if window:
+        vc[:pos0 + 4 - window + 1] = np.inf  # before the windows of rows 4 and on
+        kc[:pos0 + 4 - window + 1] = np.nan
+        clean = clean[4:]
+    vc[pos0 + m - 2:] = np.nan  # held by the last two rows only
+    kc[pos0 + m - 1:] = np.inf
+    got = aotk.attention(q, kc.reshape(-1), vc.reshape(-1), nh, nkv, hd, ctx, 0, pos0, m, window)
+    assert same_bits(got.reshape(m, -1)[clean], want.reshape(m, -1)[clean])
