@@ -200,6 +200,12 @@ void launch_sample(const SampleArgs &p, hipStream_t s);
 bool launch_matvec_quant(const DevWeight &w, const float *x, float *y, const float *add, hipStream_t s);
 void launch_matvec_multi(int n, const DevWeight *const ws[], float *const ys[], const void *x_act, size_t m,
                          hipStream_t s);
+// One token, up to three matrices of one kind and width, the input in the
+// reference's Q8_K / Q8_0 blocks (read by the matvec itself: no staging
+// launch). Returns false (nothing launched) for float kinds, K-quant rows of
+// more than 64 super-blocks, Q8_0-family rows of more than 16384 columns and
+// an output that overlaps the input.
+bool launch_matvec_blocks(int n, const DevWeight *const ws[], float *const ys[], const void *x_blocks, hipStream_t s);
 // Matrices of a Q4_K/Q5_K kind (up to three, e.g. q and k) and one Q6_K
 // matrix (e.g. v) with <= 64 super-blocks per row, same input, one launch.
 bool matvec_pair_ok(const DevWeight &a, const DevWeight &b);

@@ -67,6 +67,21 @@ struct MvArgs {
     const float *xq_src;
 };
 
+// Where a one-token matvec takes its activation from: the staged planes (xq,
+// xd, xbs), f32 (xq_src, quantized by every block), or the caller's Q8_K /
+// Q8_0 blocks as they are (xq points at them, 4-byte aligned).
+enum MvSrc { SRC_PLANES = 0, SRC_F32 = 1, SRC_BLOCKS = 2 };
+typedef unsigned u4_unal __attribute__((ext_vector_type(4), aligned(4)));
+__device__ __forceinline__ uint4 ld16(const void *p) {
+    const u4_unal v = *(const u4_unal *)p;
+    return make_uint4(v[0], v[1], v[2], v[3]);
+}
+// 16-byte piece i of the quants, piece i of the bsums and the scale of block
+// b of Q8_K blocks; piece i and scale b of Q8_0 blocks.
+__device__ __forceinline__ uint4 q8k_qs16(const void *x, int i) { return ld16(((const aotk_block_q8_k *)x)[i >> 4].qs + 16 * (i & 15)); }
+__device__ __forceinline__ uint4 q8k_bs16(const void *x, int i) { return ld16(((const aotk_block_q8_k *)x)[i >> 1].bsums + 8 * (i & 1)); }
+__device__ __forceinline__ uint4 q80_qs16(const void *x, int i) { return ld16(((const aotk_block_q8_0 *)x)[i >> 1].qs + 16 * (i & 1)); }
+
 // Ties v to this point of the program: loads before it stay before it and
 // uses of v stay after it (a volatile asm with a memory clobber).
 __device__ __forceinline__ void pin_after_loads(float4 &v) {
@@ -449,7 +464,7 @@ __host__ __device__ constexpr int kq_spl(int nb) { return nb > 0 && nb <= 32 ? 2
 // NB > 0: the super-blocks per row as a compile-time constant (immediate
 // chunk offsets, constant row-slot division, an unmasked fold); NB == 0 reads
 // it from the arguments.
-template <int KIND, int PF, int NB, bool QSRC = false>
+template <int KIND, int PF, int NB, int SRC = SRC_PLANES>
 __device__ __forceinline__ void mv_kq_body(const MvArgs &a, int RL, int G, int bx, uint8_t *sY, float (*sT)[256 + 16]) {
     using Geo = KqGeom<KIND>;
     constexpr int SPL = kq_spl(NB);
@@ -488,12 +503,17 @@ __device__ __forceinline__ void mv_kq_body(const MvArgs &a, int RL, int G, int b
     // quads of qs, one of bsums and one scale per thread; indices past the
     // end repeat the last element), then the weights of the first group:
     // waiting for the activation then leaves the weights in flight.
-    constexpr bool stage = !QSRC;  // QSRC: the input arrives in f32 (a.xq_src) and is quantized here
+    constexpr bool stage = SRC != SRC_F32;
     const int nq = nb * 16;
     uint4 xv[4], bv;
     float dv;
     float4 xf[4];  // the f32 input of the wave's first four super-blocks, when it quantizes
-    if constexpr (stage) {
+    if constexpr (SRC == SRC_BLOCKS) {
+#pragma unroll
+        for (int k = 0; k < 4; k++) xv[k] = q8k_qs16(a.xq, min(tid + 256 * k, nq - 1));
+        bv = q8k_bs16(a.xq, min(tid, 2 * nb - 1));
+        dv = ((const aotk_block_q8_k *)a.xq)[min(tid, nb - 1)].d;
+    } else if constexpr (stage) {
         const uint4 *xq = (const uint4 *)(a.xq + (size_t)tok * a.cols);
         const uint4 *xb = (const uint4 *)(a.xbs + (size_t)tok * nb * 16);
 #pragma unroll
@@ -610,10 +630,10 @@ struct KqShared {
     __align__(16) float t[4][256 + 16];  // [wave][row slot * ts + super-block] (+ read slack)
 };
 
-template <int KIND, int PF, int NB, bool QSRC = false>
+template <int KIND, int PF, int NB, int SRC = SRC_PLANES>
 __global__ __launch_bounds__(256, PF ? 2 : 4) void k_mv_kq(MvArgs a, int RL, int G) {
     __shared__ KqShared<NB> sh;
-    mv_kq_body<KIND, PF, NB, QSRC>(a, RL, G, blockIdx.x, sh.y, sh.t);
+    mv_kq_body<KIND, PF, NB, SRC>(a, RL, G, blockIdx.x, sh.y, sh.t);
 }
 
 // Two K-quant matrices of different kinds sharing the input in one launch
@@ -633,7 +653,7 @@ __global__ __launch_bounds__(256, PF ? 2 : 4) void k_mv_kq2(MvArgs a, int RLa, i
 // lane folds the row in super-block order. Half the per-lane work of one
 // lane per whole super-block, on twice the waves (Q6_K 4096x14336: 11.9
 // against 13.5 us).
-template <int KIND, int NB>
+template <int KIND, int NB, int SRC = SRC_PLANES>
 __global__ __launch_bounds__(256) void k_mv_kqw(MvArgs a) {
     static_assert(NB > 32 && NB <= 64, "rows of 33..64 super-blocks");
     __shared__ __align__(16) uint8_t sY[NB * KQ_REC];
@@ -657,9 +677,9 @@ __global__ __launch_bounds__(256) void k_mv_kqw(MvArgs a) {
     const uint4 *xb = (const uint4 *)(a.xbs + (size_t)tok * NB * 16);
     uint4 xv[4];
 #pragma unroll
-    for (int k = 0; k < 4; k++) xv[k] = xq[min(tid + 256 * k, nq - 1)];
-    const uint4 bv = xb[min(tid, 2 * NB - 1)];
-    const float dv = a.xd[(size_t)tok * NB + min(tid, NB - 1)];
+    for (int k = 0; k < 4; k++) xv[k] = SRC == SRC_BLOCKS ? q8k_qs16(a.xq, min(tid + 256 * k, nq - 1)) : xq[min(tid + 256 * k, nq - 1)];
+    const uint4 bv = SRC == SRC_BLOCKS ? q8k_bs16(a.xq, min(tid, 2 * NB - 1)) : xb[min(tid, 2 * NB - 1)];
+    const float dv = SRC == SRC_BLOCKS ? ((const aotk_block_q8_k *)a.xq)[min(tid, NB - 1)].d : a.xd[(size_t)tok * NB + min(tid, NB - 1)];
     // rows past the end load row 0 (valid memory); they are never stored
     int local;
     const int sg = seg_of(a, row_on ? row : 0, local);
@@ -1478,7 +1498,7 @@ struct Q8bW {
     uint16_t d;
 };
 
-template <int KIND, bool XQ = false, bool RUNS = KIND == AOTK_Q8_0>
+template <int KIND, int SRC = SRC_PLANES, bool RUNS = KIND == AOTK_Q8_0>
 __global__ __launch_bounds__(256) void k_mv_q8b(MvArgs a) {
     constexpr int R = Q8B_R;
     // the activation (cols int8 quants, then cols / 32 scales), sized by the
@@ -1540,15 +1560,17 @@ __global__ __launch_bounds__(256) void k_mv_q8b(MvArgs a) {
     // first two steps' weights: the wait for the activation leaves those in
     // flight
     Q8bW<KIND> cur[R], nxt[R];
-    if constexpr (!XQ) {
+    if constexpr (SRC != SRC_F32) {
         const uint4 *xq = (const uint4 *)(a.xq + (size_t)tok * a.cols);
         const int nq = (int)(a.cols / 16);
         uint4 xv[4];
 #pragma unroll
-        for (int k = 0; k < 4; k++) xv[k] = xq[min(tid + 256 * k, nq - 1)];
+        for (int k = 0; k < 4; k++) xv[k] = SRC == SRC_BLOCKS ? q80_qs16(a.xq, min(tid + 256 * k, nq - 1)) : xq[min(tid + 256 * k, nq - 1)];
         float xdv[2];
 #pragma unroll
-        for (int k = 0; k < 2; k++) xdv[k] = a.xd[(size_t)tok * nb + min(tid + 256 * k, nb - 1)];
+        for (int k = 0; k < 2; k++)
+            xdv[k] = SRC == SRC_BLOCKS ? ((const aotk_block_q8_0 *)a.xq)[min(tid + 256 * k, nb - 1)].d
+                                       : a.xd[(size_t)tok * nb + min(tid + 256 * k, nb - 1)];
         load(cur, 0);
         load(nxt, 64);
         // (unconditional stores: past the end they repeat the last element's
@@ -2549,16 +2571,18 @@ static void kq_shape(const MvArgs &a, int &RL, int &G, int &blocks) {
     blocks = (groups + 3) / 4;
 }
 
-template <int KIND>
+template <int KIND, int SRC>
 static void launch_kq(const MvArgs &a, dim3 grid, hipStream_t s) {
     // Q6_K rows of 40..56 super-blocks: two waves per row (the lighter
     // Q4_K / Q5_K terms measured faster on one lane per super-block)
-    if (KIND == AOTK_Q6_K && !a.xq_src && (a.nb == 40 || a.nb == 48 || a.nb == 56)) {
-        grid.x = (unsigned)((a.total_rows + 1) / 2);
-        if (a.nb == 40) k_mv_kqw<KIND, 40><<<grid, 256, 0, s>>>(a);
-        else if (a.nb == 48) k_mv_kqw<KIND, 48><<<grid, 256, 0, s>>>(a);
-        else k_mv_kqw<KIND, 56><<<grid, 256, 0, s>>>(a);
-        return;
+    if constexpr (KIND == AOTK_Q6_K && SRC != SRC_F32) {
+        if (a.nb == 40 || a.nb == 48 || a.nb == 56) {
+            grid.x = (unsigned)((a.total_rows + 1) / 2);
+            if (a.nb == 40) k_mv_kqw<KIND, 40, SRC><<<grid, 256, 0, s>>>(a);
+            else if (a.nb == 48) k_mv_kqw<KIND, 48, SRC><<<grid, 256, 0, s>>>(a);
+            else k_mv_kqw<KIND, 56, SRC><<<grid, 256, 0, s>>>(a);
+            return;
+        }
     }
     if (a.nb <= 64) {
         int RL, G, blocks;
@@ -2568,27 +2592,36 @@ static void launch_kq(const MvArgs &a, dim3 grid, hipStream_t s) {
         // except for Q6_K rows of one lane per super-block, measured faster
         // with the loads of a second register set in flight
         const bool pf0 = G == 1 && !(KIND == AOTK_Q6_K && kq_spl(a.nb) == 1);
-        if (a.xq_src && pf0) {
-#define F(NB) k_mv_kq<KIND, 0, NB, true><<<grid, 256, 0, s>>>(a, RL, G)
-            AOTK_NB_SWITCH(a.nb, F)
-#undef F
-        } else if (a.xq_src) {
-#define F(NB) k_mv_kq<KIND, 1, NB, true><<<grid, 256, 0, s>>>(a, RL, G)
-            AOTK_NB_SWITCH(a.nb, F)
-#undef F
-        } else if (pf0) {
-#define F(NB) k_mv_kq<KIND, 0, NB><<<grid, 256, 0, s>>>(a, RL, G)
+        if (pf0) {
+#define F(NB) k_mv_kq<KIND, 0, NB, SRC><<<grid, 256, 0, s>>>(a, RL, G)
             AOTK_NB_SWITCH(a.nb, F)
 #undef F
         } else {
-#define F(NB) k_mv_kq<KIND, 1, NB><<<grid, 256, 0, s>>>(a, RL, G)
+#define F(NB) k_mv_kq<KIND, 1, NB, SRC><<<grid, 256, 0, s>>>(a, RL, G)
             AOTK_NB_SWITCH(a.nb, F)
 #undef F
         }
-    } else {
+    } else if constexpr (SRC == SRC_PLANES) {
         grid.x = (unsigned)((a.total_rows + 7) / 8);
         k_mv_kquant<KIND, 2><<<grid, 256, 0, s>>>(a);
     }
+}
+
+template <int SRC>
+static void launch_kq(int kind, const MvArgs &a, dim3 grid, hipStream_t s) {
+    if (kind == AOTK_Q4_K) launch_kq<AOTK_Q4_K, SRC>(a, grid, s);
+    else if (kind == AOTK_Q5_K) launch_kq<AOTK_Q5_K, SRC>(a, grid, s);
+    else launch_kq<AOTK_Q6_K, SRC>(a, grid, s);
+}
+
+// cols <= Q8B_MAX_COLS
+template <int SRC>
+static void launch_q8b(int kind, const MvArgs &a, dim3 grid, hipStream_t s) {
+    grid.x = (unsigned)((a.total_rows + 4 * Q8B_R - 1) / (4 * Q8B_R));
+    if (kind == AOTK_Q8_0 && a.total_rows >= 65536 && SRC != SRC_F32) k_mv_q8b<AOTK_Q8_0, SRC, false><<<grid, 256, q8b_lds(a), s>>>(a);
+    else if (kind == AOTK_Q8_0) k_mv_q8b<AOTK_Q8_0, SRC><<<grid, 256, q8b_lds(a), s>>>(a);
+    else if (kind == AOTK_Q4_0) k_mv_q8b<AOTK_Q4_0, SRC><<<grid, 256, q8b_lds(a), s>>>(a);
+    else k_mv_q8b<AOTK_Q5_0, SRC><<<grid, 256, q8b_lds(a), s>>>(a);
 }
 
 // Persistent k_mm_kx: one round of resident blocks (the occupancy of the
@@ -2683,41 +2716,21 @@ static void launch_args(int kind, const MvArgs &a, size_t m, hipStream_t s) {
     }
     switch (kind) {
     case AOTK_Q4_K:
-        launch_kq<AOTK_Q4_K>(a, grid, s);
-        break;
     case AOTK_Q5_K:
-        launch_kq<AOTK_Q5_K>(a, grid, s);
-        break;
     case AOTK_Q6_K:
-        launch_kq<AOTK_Q6_K>(a, grid, s);
+        launch_kq<SRC_PLANES>(kind, a, grid, s);
         break;
     case AOTK_Q8_0:
-        if (a.cols <= (size_t)Q8B_MAX_COLS) {
-            grid.x = (unsigned)((a.total_rows + 4 * Q8B_R - 1) / (4 * Q8B_R));
-            if (a.total_rows >= 65536) k_mv_q8b<AOTK_Q8_0, false, false><<<grid, 256, q8b_lds(a), s>>>(a);
-            else k_mv_q8b<AOTK_Q8_0><<<grid, 256, q8b_lds(a), s>>>(a);
-        } else {
-            grid.x = (unsigned)((a.total_rows + 31) / 32);
-            k_mv_q80<AOTK_Q8_0><<<grid, 256, 0, s>>>(a);
-        }
-        break;
     case AOTK_Q4_0:
-        if (a.cols <= (size_t)Q8B_MAX_COLS) {
-            grid.x = (unsigned)((a.total_rows + 4 * Q8B_R - 1) / (4 * Q8B_R));
-            k_mv_q8b<AOTK_Q4_0><<<grid, 256, q8b_lds(a), s>>>(a);
-        } else {
-            grid.x = (unsigned)((a.total_rows + 31) / 32);
-            k_mv_q80<AOTK_Q4_0><<<grid, 256, 0, s>>>(a);
-        }
-        break;
     case AOTK_Q5_0:
         if (a.cols <= (size_t)Q8B_MAX_COLS) {
-            grid.x = (unsigned)((a.total_rows + 4 * Q8B_R - 1) / (4 * Q8B_R));
-            k_mv_q8b<AOTK_Q5_0><<<grid, 256, q8b_lds(a), s>>>(a);
-        } else {
-            grid.x = (unsigned)((a.total_rows + 31) / 32);
-            k_mv_q80<AOTK_Q5_0><<<grid, 256, 0, s>>>(a);
+            launch_q8b<SRC_PLANES>(kind, a, grid, s);
+            break;
         }
+        grid.x = (unsigned)((a.total_rows + 31) / 32);
+        if (kind == AOTK_Q8_0) k_mv_q80<AOTK_Q8_0><<<grid, 256, 0, s>>>(a);
+        else if (kind == AOTK_Q4_0) k_mv_q80<AOTK_Q4_0><<<grid, 256, 0, s>>>(a);
+        else k_mv_q80<AOTK_Q5_0><<<grid, 256, 0, s>>>(a);
         break;
     case AOTK_F16:
     case AOTK_BF16: {
@@ -2772,10 +2785,7 @@ bool launch_matvec_quant(const DevWeight &w, const float *x, float *y, const flo
         ActQ8_0 none = {};
         MvArgs a = make_args(1, ws, ys, adds, &none);
         a.xq_src = x;
-        const dim3 grid((unsigned)((a.total_rows + 4 * Q8B_R - 1) / (4 * Q8B_R)), 1);
-        if (kind == AOTK_Q8_0) k_mv_q8b<AOTK_Q8_0, true><<<grid, 256, q8b_lds(a), s>>>(a);
-        else if (kind == AOTK_Q4_0) k_mv_q8b<AOTK_Q4_0, true><<<grid, 256, q8b_lds(a), s>>>(a);
-        else k_mv_q8b<AOTK_Q5_0, true><<<grid, 256, q8b_lds(a), s>>>(a);
+        launch_q8b<SRC_F32>(kind, a, dim3(1, 1), s);
         return true;
     }
     if ((kind != AOTK_Q4_K && kind != AOTK_Q5_K && kind != AOTK_Q6_K) || w.nb > 64)
@@ -2783,10 +2793,36 @@ bool launch_matvec_quant(const DevWeight &w, const float *x, float *y, const flo
     ActQ8K none = {};
     MvArgs a = make_args(1, ws, ys, adds, &none);
     a.xq_src = x;
-    dim3 grid(1, 1);
-    if (kind == AOTK_Q4_K) launch_kq<AOTK_Q4_K>(a, grid, s);
-    else if (kind == AOTK_Q5_K) launch_kq<AOTK_Q5_K>(a, grid, s);
-    else launch_kq<AOTK_Q6_K>(a, grid, s);
+    launch_kq<SRC_F32>(kind, a, dim3(1, 1), s);
+    return true;
+}
+
+// Bound by latency, not bytes: of a call's ~20 us the matvec is 7..12, and the
+// staging launch with its gap was another 3.2. The planes it wrote differ from
+// the blocks only in where a super-block's quants, bsums and scale lie, and
+// every block of the matvec copies the whole input to LDS anyway, so the blocks
+// are read there: 4-byte aligned 16-byte loads, from L2 after the first reader.
+// Calls of 14336x4096 Q4_K 20.8 -> 17.6 us, 4096x12288 Q8_0 25.4 -> 22.4 us.
+// Longer rows stay on the staged planes: their kernels re-read the input from
+// memory and not from LDS. So does a whole forward pass, which quantizes where
+// it produces the input and has no blocks.
+bool launch_matvec_blocks(int n, const DevWeight *const ws[], float *const ys[], const void *x_blocks, hipStream_t s) {
+    const int kind = ws[0]->kind, act = activation(kind);
+    if (act == ACT_F32 || (uintptr_t)x_blocks % 4 != 0) return false;
+    if (act == ACT_Q8_K ? ws[0]->nb > 64 : ws[0]->cols > (size_t)Q8B_MAX_COLS) return false;
+    // an output laid over the input needs the staged copy: here one block may
+    // store its rows before another has read the input
+    const uintptr_t x0 = (uintptr_t)x_blocks;
+    const uintptr_t x1 = x0 + (act == ACT_Q8_K ? ws[0]->cols / 256 * sizeof(aotk_block_q8_k)
+                                               : ws[0]->cols / 32 * sizeof(aotk_block_q8_0));
+    for (int i = 0; i < n; i++)
+        if ((uintptr_t)ys[i] < x1 && x0 < (uintptr_t)(ys[i] + ws[i]->rows)) return false;
+    ActQ8K qk = {};
+    ActQ8_0 q0 = {};
+    MvArgs a = make_args(n, ws, ys, nullptr, act == ACT_Q8_K ? (const void *)&qk : (const void *)&q0);
+    a.xq = (const int8_t *)x_blocks;
+    if (act == ACT_Q8_K) launch_kq<SRC_BLOCKS>(kind, a, dim3(1, 1), s);
+    else launch_q8b<SRC_BLOCKS>(kind, a, dim3(1, 1), s);
     return true;
 }
 

@@ -321,11 +321,15 @@ int aotk_matvec(const aotk_weight *w, const void *x_dev, float *out_dev) { retur
 int aotk_matmul(const aotk_weight *w, const void *xs_dev, size_t m, float *out_dev) {
     if (!w) return fail("null weight");
     if (m == 0) return 0;
-    ActQ8K qk;
-    ActQ8_0 q0;
-    const void *act;
-    if (stage_act(w->dw, xs_dev, m, qk, q0, act)) return -1;
-    launch_matvec(w->dw, act, m, out_dev, nullptr, g_stream);
+    const DevWeight *dws[1] = {&w->dw};
+    float *ys[1] = {out_dev};
+    if (!(m == 1 && launch_matvec_blocks(1, dws, ys, xs_dev, g_stream))) {
+        ActQ8K qk;
+        ActQ8_0 q0;
+        const void *act;
+        if (stage_act(w->dw, xs_dev, m, qk, q0, act)) return -1;
+        launch_matvec(w->dw, act, m, out_dev, nullptr, g_stream);
+    }
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(g_stream));
     return 0;
@@ -344,17 +348,19 @@ static int multi_product(int n, const aotk_weight *const *ws, const void *xs_dev
             return fail("%s: the matrices differ in kind or shape", what);
     }
     if (m == 0) return 0;
-    ActQ8K qk;
-    ActQ8_0 q0;
-    const void *act;
-    if (stage_act(w0, xs_dev, m, qk, q0, act)) return -1;
     const DevWeight *dws[3];
     float *ys[3];
     for (int i = 0; i < n; i++) {
         dws[i] = &ws[i]->dw;
         ys[i] = outs[i];
     }
-    launch_matvec_multi(n, dws, ys, act, m, g_stream);
+    if (!(m == 1 && launch_matvec_blocks(n, dws, ys, xs_dev, g_stream))) {
+        ActQ8K qk;
+        ActQ8_0 q0;
+        const void *act;
+        if (stage_act(w0, xs_dev, m, qk, q0, act)) return -1;
+        launch_matvec_multi(n, dws, ys, act, m, g_stream);
+    }
     HIPC(hipGetLastError());
     HIPC(hipStreamSynchronize(g_stream));
     return 0;

@@ -128,3 +128,34 @@ def test_prompt_attention_masks_positions(aotk, oracle, nh, nkv, hd, pos0, m, wi
     kc[pos0 + m - 1:] = np.inf
     got = aotk.attention(q, kc.reshape(-1), vc.reshape(-1), nh, nkv, hd, ctx, 0, pos0, m, window)
     assert same_bits(got.reshape(m, -1)[clean], want.reshape(m, -1)[clean])
+
+
+@pytest.mark.parametrize("kind,cols", [(Q4_K, 256), (Q4_K, 2048), (Q4_K, 4096), (Q4_K, 16384), (Q4_K, 16640), (Q5_K, 2560), (Q5_K, 5632),
+                                       (Q6_K, 768), (Q6_K, 10240), (Q6_K, 12288), (Q6_K, 14336), (Q6_K, 11008),
+                                       (Q8_0, 32), (Q8_0, 4128), (Q8_0, 16384), (Q8_0, 16416), (Q4_0, 96), (Q4_0, 16384),
+                                       (Q5_0, 2080)])
+def test_matvec_from_blocks(aotk, oracle, kind, cols):
+    """One token in the reference's blocks, single and as three matrices: the
+    widths where the matvec reads the blocks itself, and the first past them."""
+    rng = np.random.default_rng(cols + kind)
+    rows = (37, 5, 70)
+    x = oracle.quantize_act(kind, (rng.standard_normal(cols) * 3).astype(np.float32))
+    raws = [oracle.quantize_rows(kind, (rng.standard_normal((r, cols)) * 0.02).astype(np.float32)) for r in rows]
+    refs = [oracle.matvec(kind, w, x, r, cols) for w, r in zip(raws, rows)]
+    ws = [aotk.Weight(kind, w, r, cols) for w, r in zip(raws, rows)]
+    assert same_bits(aotk.matvec(ws[0], x), refs[0])
+    for got, ref in zip(aotk.matvec3(ws, x), refs):
+        assert same_bits(got, ref)
+
+
+@pytest.mark.parametrize("kind", [Q4_K, Q8_0])
+def test_matvec_output_over_its_input(aotk, oracle, kind):
+    rng = np.random.default_rng(kind)
+    rows, cols = 700, 4096
+    x = oracle.quantize_act(kind, rng.standard_normal(cols).astype(np.float32))
+    raw = oracle.quantize_rows(kind, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    w = aotk.Weight(kind, raw, rows, cols)
+    buf = aotk.DeviceBuffer.from_numpy(np.ascontiguousarray(x).view(np.uint8).reshape(-1))
+    lib = aotk.runtime._lib()
+    assert lib.aotk_matvec(w.h, buf.ptr, buf.ptr) == 0
+    assert same_bits(buf.to_numpy(np.float32, rows), oracle.matvec(kind, raw, x, rows, cols))
