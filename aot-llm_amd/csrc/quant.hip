@@ -430,15 +430,27 @@ __global__ void k_q8k_to_ref(ActQ8K a, size_t nblk, aotk_block_q8_k *out) {
     if (e < 16) out[b].bsums[e] = a.bsums[b * 16 + e];
     if (e == 0) out[b].d = a.d[b];
 }
-__global__ void k_ref_to_q8k(const aotk_block_q8_k *in, size_t nblk, ActQ8K a) {
-    size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= nblk * 256) return;
-    size_t b = i / 256;
-    int e = (int)(i % 256);
-    a.qs[i] = in[b].qs[e];
-    if (a.qt) a.qt[q8k_tiled_off(b / a.nbt, (int)(b % a.nbt), a.nbt, e)] = in[b].qs[e];
-    if (e < 16) a.bsums[b * 16 + e] = in[b].bsums[e];
-    if (e == 0) a.d[b] = in[b].d;
+// Block = (super-block, 16 vectors), thread = (step pair p, k group g, vector)
+// with the 16-byte piece of q8k_tiled_off, elements 32(2p) + 8g .. + 7 and the
+// eight 32 on: a wave's tiled stores are one kilobyte in a row. Bound by latency;
+// a byte per thread took 5.0 us for 64 vectors of 14336 (the call 52.7 us), this
+// takes 3.8 (51.4). A 16-byte piece of one vector per thread: 3.9 (51.9). (The
+// Q8_0 copy below stays at a value per thread: in pieces its launch took 3.0 us
+// against 2.8 and the product behind it up to 2 us more.)
+__global__ __launch_bounds__(256) void k_ref_to_q8k(const aotk_block_q8_k *__restrict__ in, int nb, size_t rows, ActQ8K a) {
+    const int t = threadIdx.x, sb = (int)(blockIdx.x % (unsigned)nb);
+    const size_t v0 = (size_t)(blockIdx.x / (unsigned)nb) * 16, v = v0 + (t & 15), vs = v0 + (t >> 4);
+    if (v < rows) {
+        const size_t b = v * nb + sb;
+        const int e = (t >> 6) * 64 + ((t >> 4) & 3) * 8;
+        const unsigned *q = (const unsigned *)(in[b].qs + e);
+        const uint2 lo = make_uint2(q[0], q[1]), hi = make_uint2(q[8], q[9]);
+        *(uint2 *)(a.qs + b * 256 + e) = lo;
+        *(uint2 *)(a.qs + b * 256 + e + 32) = hi;
+        if (a.qt) *(uint4 *)(a.qt + q8k_tiled_off(v, sb, nb, e)) = make_uint4(lo.x, lo.y, hi.x, hi.y);
+        if (t < 16) a.d[b] = in[b].d;
+    }
+    if (vs < rows) a.bsums[(vs * nb + sb) * 16 + (t & 15)] = in[vs * nb + sb].bsums[t & 15];
 }
 __global__ void k_q8_0_to_ref(ActQ8_0 a, size_t nblk, aotk_block_q8_0 *out) {
     size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -463,10 +475,9 @@ void launch_q8k_to_ref(ActQ8K a, size_t n, aotk_block_q8_k *out, hipStream_t s) 
     k_q8k_to_ref<<<(unsigned)((nblk * 256 + 255) / 256), 256, 0, s>>>(a, nblk, out);
 }
 void launch_ref_to_q8k(const aotk_block_q8_k *in, size_t n, size_t rows, ActQ8K a, hipStream_t s) {
-    size_t nblk = rows * n / 256;
     a.nbt = (int)(n / 256);
     if (rows < 2) a.qt = nullptr;
-    k_ref_to_q8k<<<(unsigned)((nblk * 256 + 255) / 256), 256, 0, s>>>(in, nblk, a);
+    k_ref_to_q8k<<<(unsigned)((rows + 15) / 16 * a.nbt), 256, 0, s>>>(in, a.nbt, rows, a);
 }
 void launch_q8_0_to_ref(ActQ8_0 a, size_t n, aotk_block_q8_0 *out, hipStream_t s) {
     size_t nblk = n / 32;

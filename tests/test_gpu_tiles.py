@@ -159,3 +159,15 @@ def test_matvec_output_over_its_input(aotk, oracle, kind):
     lib = aotk.runtime._lib()
     assert lib.aotk_matvec(w.h, buf.ptr, buf.ptr) == 0
     assert same_bits(buf.to_numpy(np.float32, rows), oracle.matvec(kind, raw, x, rows, cols))
+
+
+@pytest.mark.parametrize("kind,rows,cols,m", [(Q4_K, 2048, 256, 2), (Q6_K, 2050, 768, 17), (Q5_K, 100, 2304, 33), (Q4_K, 33, 512, 16)])
+def test_kquant_staging_tiles(aotk, oracle, kind, rows, cols, m):
+    """The staged copies of the input's blocks (tiled and plain) around whole
+    and partial 16-vector tiles."""
+    rng = np.random.default_rng(rows + m)
+    xs = np.concatenate([np.ascontiguousarray(oracle.quantize_act(kind, rng.standard_normal(cols).astype(np.float32))).view(np.uint8).reshape(-1)
+                         for _ in range(m)])
+    raw = oracle.quantize_rows(kind, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
+    got = aotk.matmul(aotk.Weight(kind, raw, rows, cols), xs, m)
+    assert same_bits(got, oracle.matmul(kind, raw, xs, m, rows, cols, pool=oracle.Pool(8)).reshape(m, rows))
