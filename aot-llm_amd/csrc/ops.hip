@@ -42,66 +42,10 @@ __device__ float block_sum(float v, float *red) {
     return t;
 }
 
-// Sequential f32 sum of n LDS values in index order, by one thread.
-// Plain sums run through lds_chain128 in runs of 128; the rest (and the sums
-// of squares) in groups of 32 that alternate between two register sets with
-// no copies between them: the reads of the next group are issued before the
-// adds of the current one (unconditionally: past the last full group they
-// re-read it). v 16-byte aligned.
-template <bool SQUARE>
-__device__ __forceinline__ float seq_sum_lds(const float *v, int n) {
-    float s = 0.0f;
-    int i = 0;
-    if (!SQUARE)
-        for (; i + 128 <= n; i += 128) s = lds_chain128(v + i, s);
-    const int nfull = i + (n - i) / 32 * 32;
-    auto add = [&](const float4 (&g)[8]) {
-#pragma unroll
-        for (int k = 0; k < 8; k++) {
-            if (SQUARE) {
-                s += g[k].x * g[k].x;
-                s += g[k].y * g[k].y;
-                s += g[k].z * g[k].z;
-                s += g[k].w * g[k].w;
-            } else {
-                s += g[k].x;
-                s += g[k].y;
-                s += g[k].z;
-                s += g[k].w;
-            }
-        }
-    };
-    if (nfull > i) {
-        const int last = nfull - 32;
-        float4 a[8], b[8];
-#pragma unroll
-        for (int k = 0; k < 8; k++) a[k] = *(const float4 *)(v + i + 4 * k);
-        for (;;) {
-#pragma unroll
-            for (int k = 0; k < 8; k++) b[k] = *(const float4 *)(v + min(i + 32, last) + 4 * k);
-            add(a);
-            i += 32;
-            if (i >= nfull) break;
-#pragma unroll
-            for (int k = 0; k < 8; k++) a[k] = *(const float4 *)(v + min(i + 32, last) + 4 * k);
-            add(b);
-            i += 32;
-            if (i >= nfull) break;
-        }
-    }
-    for (; i < n; i++) s += SQUARE ? v[i] * v[i] : v[i];
-    return s;
-}
-
-// The same for v padded with -0.0 up to a multiple of 64 values: whole
-// runs of the assembly chain.
+// Sequential f32 sum of n LDS values in index order, by one thread: v 16-byte
+// aligned and padded with -0.0 up to a multiple of 64 values.
 __device__ __forceinline__ float seq_sum_lds_pad64(const float *v, int n) {
-    const int n64 = (n + 63) & ~63;
-    float s = 0.0f;
-    int i = 0;
-    for (; i + 128 <= n64; i += 128) s = lds_chain128(v + i, s);
-    if (i < n64) s = lds_chain64(v + i, s);
-    return s;
+    return lds_chain(v, (n + 63) >> 6, 0.0f);
 }
 
 // ss = sum of v*v over n <= 256 values in LDS, in index order
@@ -758,8 +702,8 @@ __global__ __launch_bounds__(HD == 256 ? 64 * (QKD_MAX_GQA_256 + 1) : 576) void 
 //   output (ops.rs:209-215): chunks of CP positions: all threads form the
 //   products p_t * v_t,d into LDS, dim-major (row of dim d: CP products and
 //   4 pad floats), with the float4 V loads issued PD chunks ahead; then
-//   thread d adds its row in position order (lds_chain) while the others
-//   form the next chunk. Sixteen dims per block put 8 blocks on every head
+//   thread d adds its row in position order (lds_chain_chunks384, which does
+//   not stop between chunks) while the others form the next chunk. Sixteen dims per block put 8 blocks on every head
 //   (256 for 32 heads); chunks of 384 positions halve the barriers per
 //   position against 192.
 #ifndef ATT_TS
@@ -779,8 +723,8 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_sv(AttnArgs a) {
     constexpr int DB = SV_DB;
     constexpr int CP = SV_CP;
     __shared__ __align__(16) float e[SEQ_PAD_N > ATT_MAX_SPAN + 64 ? SEQ_PAD_N : ATT_MAX_SPAN + 64];
-    // product buffers (+64 floats read past the end by the last groups) / sum scratch
-    __shared__ __align__(16) uint8_t ubuf[sizeof(SeqScratch) > (2 * SV_BUF + 64) * 4 ? sizeof(SeqScratch) : (2 * SV_BUF + 64) * 4];
+    // product buffers / sum scratch
+    __shared__ __align__(16) uint8_t ubuf[sizeof(SeqScratch) > 2 * SV_BUF * 4 ? sizeof(SeqScratch) : 2 * SV_BUF * 4];
     __shared__ float red[SEQ_T / 64];
     __shared__ float bc;
     __shared__ uint64_t stab[32];  // expf's 2^(i/32) table
@@ -805,7 +749,7 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_sv(AttnArgs a) {
     // are dealt to the 4 SIMDs in turn) form them, so the dependent adds
     // issue back to back
     constexpr int NPROD = (SEQ_T / 64 - SEQ_T / 256) * 64;
-    static_assert(CP == 384, "the output adds of a full chunk run in lds_chain384");
+    static_assert(CP == 384, "the output adds run in lds_chain_chunks384");
     static_assert(CP * R4 == 2 * NPROD, "two float4 per producer thread per chunk");
     // V loads run PD chunks ahead of the products (a register ring)
     constexpr int PD = 8;
@@ -872,44 +816,38 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_sv(AttnArgs a) {
     if (pid >= 0)
 #pragma unroll
         for (int j = PE; j < PD; j++) issue(ring[j], j);
-    for (int c0 = 0; c0 < nch; c0 += PD) {
+    // (a wave either adds or forms products; both sides meet nch barriers)
+    if (__builtin_amdgcn_readfirstlane(wv) == 0) {
+        if (tid < DB) o = lds_chain_chunks384(prod + tid * SV_RS, prod + SV_BUF + tid * SV_RS, (cnt + 63) >> 6, 0.0f);
+    } else {
+        for (int c0 = 0; c0 < nch; c0 += PD) {
 #pragma unroll
-        for (int j = 0; j < PD; j++) {
-            const int c = c0 + j;
-            if (c < nch) {
-                float *buf = prod + (c & 1) * SV_BUF;
-                const int base = c * CP;
-                const int rows = min(CP, cnt - base);
-                if (pid >= 0) {
+            for (int j = 0; j < PD; j++) {
+                const int c = c0 + j;
+                if (c < nch) {
+                    float *buf = prod + (c & 1) * SV_BUF;
+                    const int base = c * CP;
+                    const int rows = min(CP, cnt - base);
+                    if (pid >= 0) {
 #pragma unroll
-                    for (int k = 0; k < 2; k++) {
-                        const int idx = pid + k * NPROD;
-                        const int r = idx / R4, d = 4 * (idx % R4);
-                        // rows past the span hold -0.0, which leaves any sum unchanged
-                        const bool in = r < rows;
-                        const float pt = in ? e[at(base + r)] : 0.0f;
-                        const float4 v4 = ring[j][k];
-                        buf[(d + 0) * SV_RS + r] = in ? pt * v4.x : -0.0f;
-                        buf[(d + 1) * SV_RS + r] = in ? pt * v4.y : -0.0f;
-                        buf[(d + 2) * SV_RS + r] = in ? pt * v4.z : -0.0f;
-                        buf[(d + 3) * SV_RS + r] = in ? pt * v4.w : -0.0f;
+                        for (int k = 0; k < 2; k++) {
+                            const int idx = pid + k * NPROD;
+                            const int r = idx / R4, d = 4 * (idx % R4);
+                            // rows past the span hold -0.0, which leaves any sum unchanged
+                            const bool in = r < rows;
+                            const float pt = in ? e[at(base + r)] : 0.0f;
+                            const float4 v4 = ring[j][k];
+                            buf[(d + 0) * SV_RS + r] = in ? pt * v4.x : -0.0f;
+                            buf[(d + 1) * SV_RS + r] = in ? pt * v4.y : -0.0f;
+                            buf[(d + 2) * SV_RS + r] = in ? pt * v4.z : -0.0f;
+                            buf[(d + 3) * SV_RS + r] = in ? pt * v4.w : -0.0f;
+                        }
+                        issue(ring[j], c + PD);
                     }
-                    issue(ring[j], c + PD);
+                    SV_TS(c, 0);
+                    __syncthreads();
+                    SV_TS(c, 1);
                 }
-                SV_TS(c, 0);
-                __syncthreads();
-                SV_TS(c, 1);
-                if (tid < DB) {
-                    // the chunk's rows rounded up to 64 (the padding adds -0.0)
-                    const float *tp = buf + tid * SV_RS;
-                    if (rows > 320) o = lds_chain384(tp, o);
-                    else if (rows > 256) o = lds_chain128(tp + 192, lds_chain192(tp, o));
-                    else if (rows > 192) o = lds_chain256(tp, o);
-                    else if (rows > 128) o = lds_chain192(tp, o);
-                    else if (rows > 64) o = lds_chain128(tp, o);
-                    else o = lds_chain64(tp, o);
-                }
-                SV_TS(c, 2);
             }
         }
     }
@@ -942,7 +880,7 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_decode1(AttnArgs a, QkvPost p) {
     // scores / exps, padded to a run of 64 (spans below SV_SEQ_MIN: the one-thread sum)
     static_assert(AD_MAX_SPAN < SV_SEQ_MIN && AD_MAX_SPAN <= SEQ_T, "one position per thread, the one-thread sum");
     __shared__ __align__(16) float e[AD_MAX_SPAN + 64];
-    __shared__ __align__(16) float prod[2 * SV_BUF + 64];  // product buffers (+64 floats read past the end by the last groups)
+    __shared__ __align__(16) float prod[SV_BUF];
     __shared__ float red[SEQ_T / 64];
     __shared__ float bc;
     __shared__ uint64_t stab[32];  // expf's 2^(i/32) table
@@ -976,22 +914,16 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_decode1(AttnArgs a, QkvPost p) {
         }
     constexpr int R4 = DB / 4;
     constexpr int NPROD = (SEQ_T / 64 - SEQ_T / 256) * 64;
-    static_assert(CP * R4 == 2 * NPROD, "two float4 per producer thread per chunk");
-    constexpr int PD = 8;
-    float4 ring[PD][2];
+    static_assert(CP * R4 == 2 * NPROD && AD_MAX_SPAN <= CP, "one chunk, two float4 per producer thread");
     const int pid = (wv & 3) ? (wv - (wv >> 2) - 1) * 64 + lane : -1;
-    auto issue = [&](float4 (&dst)[2], int c) {
+    float4 vin[2];  // in flight through the softmax
+    if (pid >= 0)
 #pragma unroll
         for (int k = 0; k < 2; k++) {
             const int idx = pid + k * NPROD;
-            const int t = c * CP + idx / R4;
-            dst[k] = t < cnt ? *(const float4 *)(vb + (size_t)t * kv + 4 * (idx % R4)) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+            const int t = idx / R4;
+            vin[k] = t < cnt ? *(const float4 *)(vb + (size_t)t * kv + 4 * (idx % R4)) : make_float4(0.0f, 0.0f, 0.0f, 0.0f);
         }
-    };
-    constexpr int PE = 2;
-    if (pid >= 0)
-#pragma unroll
-        for (int j = 0; j < PE; j++) issue(ring[j], j);
     exp_table_to_lds(stab);
     if (wv == 0) head_post_wave<HD>(hq, htmp[0], hin, p.bq != nullptr, p.q_norm != nullptr, (int)p.rot_dim, p.neox, p.eps);
     else if (wv == 1) head_post_wave<HD>(hk, htmp[1], hin, p.bk != nullptr, p.k_norm != nullptr, (int)p.rot_dim, p.neox, p.eps);
@@ -1034,49 +966,23 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_decode1(AttnArgs a, QkvPost p) {
     const float inv = 1.0f / sum;
     for (int t = tid; t < cnt; t += SEQ_T) e[at(t)] = e[at(t)] * inv;
     __syncthreads();  // the sum's scratch is reused for the products below
-    float o = 0.0f;
-    const int nch = (cnt + CP - 1) / CP;
-    if (pid >= 0)
+    if (pid >= 0) {
 #pragma unroll
-        for (int j = PE; j < PD; j++) issue(ring[j], j);
-    for (int c0 = 0; c0 < nch; c0 += PD) {
-#pragma unroll
-        for (int j = 0; j < PD; j++) {
-            const int c = c0 + j;
-            if (c < nch) {
-                float *buf = prod + (c & 1) * SV_BUF;
-                const int base = c * CP;
-                const int rows = min(CP, cnt - base);
-                if (pid >= 0) {
-#pragma unroll
-                    for (int k = 0; k < 2; k++) {
-                        const int idx = pid + k * NPROD;
-                        const int r = idx / R4, d = 4 * (idx % R4);
-                        const bool in = r < rows;
-                        const float pt = in ? e[at(base + r)] : 0.0f;
-                        // the new position's v from LDS (its cache row may not be written yet)
-                        const float4 v4 = base + r == cnt - 1 ? *(const float4 *)(hv + d0 + d) : ring[j][k];
-                        buf[(d + 0) * SV_RS + r] = in ? pt * v4.x : -0.0f;
-                        buf[(d + 1) * SV_RS + r] = in ? pt * v4.y : -0.0f;
-                        buf[(d + 2) * SV_RS + r] = in ? pt * v4.z : -0.0f;
-                        buf[(d + 3) * SV_RS + r] = in ? pt * v4.w : -0.0f;
-                    }
-                    issue(ring[j], c + PD);
-                }
-                __syncthreads();
-                if (tid < DB) {
-                    const float *tp = buf + tid * SV_RS;
-                    if (rows > 320) o = lds_chain384(tp, o);
-                    else if (rows > 256) o = lds_chain128(tp + 192, lds_chain192(tp, o));
-                    else if (rows > 192) o = lds_chain256(tp, o);
-                    else if (rows > 128) o = lds_chain192(tp, o);
-                    else if (rows > 64) o = lds_chain128(tp, o);
-                    else o = lds_chain64(tp, o);
-                }
-            }
+        for (int k = 0; k < 2; k++) {
+            const int idx = pid + k * NPROD;
+            const int r = idx / R4, d = 4 * (idx % R4);
+            const bool in = r < cnt;
+            const float pt = in ? e[at(r)] : 0.0f;
+            // the new position's v from LDS (its cache row may not be written yet)
+            const float4 v4 = r == cnt - 1 ? *(const float4 *)(hv + d0 + d) : vin[k];
+            prod[(d + 0) * SV_RS + r] = in ? pt * v4.x : -0.0f;
+            prod[(d + 1) * SV_RS + r] = in ? pt * v4.y : -0.0f;
+            prod[(d + 2) * SV_RS + r] = in ? pt * v4.z : -0.0f;
+            prod[(d + 3) * SV_RS + r] = in ? pt * v4.w : -0.0f;
         }
     }
-    if (tid < DB) a.out[(size_t)h * HD + d0 + tid] = o;
+    __syncthreads();
+    if (tid < DB) a.out[(size_t)h * HD + d0 + tid] = lds_chain(prod + tid * SV_RS, (cnt + 63) >> 6, 0.0f);
 }
 
 // Batched rows (prompt chunks), spans up to ATT_MAX_SPAN: the same softmax

@@ -171,3 +171,17 @@ def test_kquant_staging_tiles(aotk, oracle, kind, rows, cols, m):
     raw = oracle.quantize_rows(kind, (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32))
     got = aotk.matmul(aotk.Weight(kind, raw, rows, cols), xs, m)
     assert same_bits(got, oracle.matmul(kind, raw, xs, m, rows, cols, pool=oracle.Pool(8)).reshape(m, rows))
+
+
+@pytest.mark.parametrize("hd", [64, 128, 256])
+@pytest.mark.parametrize("span", [1, 64, 65, 320, 321, 384, 385, 448, 768, 769, 1023, 1152, 1537, 4609])
+def test_decode_attention_chunks(aotk, oracle, hd, span):
+    """One row over spans around the 64-value runs and the 384-position chunks
+    of its ordered sums, signed zeros and subnormal products among them."""
+    rng = np.random.default_rng(span + hd)
+    q = rng.standard_normal(4 * hd).astype(np.float32)
+    kc, vc = (rng.standard_normal(span * 2 * hd).astype(np.float32) for _ in range(2))
+    vc[::3] = np.float32(-0.0)
+    vc[1::5] *= np.float32(1e-39)
+    got = aotk.attention(q, kc, vc, 4, 2, hd, span, 0, span - 1, 1, 0)
+    assert same_bits(got, attention_ref(oracle, q, kc, vc, 4, 2, hd, span, span - 1, 1, 0))
