@@ -369,14 +369,16 @@ __device__ __forceinline__ void row_range(const AttnArgs &a, size_t i, size_t &t
 }
 
 // Scores: block = (kv head, chunk of ATT_CH positions, row), gqa * 64
-// threads. The chunk's K rows are staged in LDS (coalesced row loads, row
-// stride HD + 1 so that lanes reading one dimension of 64 rows hit 64
-// banks); thread (query head of the group, position) then runs its dot
-// product sequentially over the head dimension.
+// threads. The chunk's K rows are staged in LDS (coalesced row loads, eight per
+// thread in flight; row stride HD + 4: 16-byte rows, the 16-byte reads of 16
+// rows hit all banks); thread (query head of the group, position) then runs its
+// dot product sequentially over the head dimension. 8 kv heads x 4100
+// positions, head_dim 128 (16.8 MB): 8.0 -> 6.7 us against one load at a time
+// and 4-byte reads.
 template <int HD>
 __global__ __launch_bounds__(512) void k_attn_scores(AttnArgs a) {
-    constexpr int KS = HD + 1;
-    __shared__ float sk[ATT_CH * KS];
+    constexpr int KS = HD + 4;
+    __shared__ __align__(16) float sk[ATT_CH * KS];
     __shared__ __align__(16) float sq[ATT_MAX_GQA][HD];
     const int gqa = a.n_head / a.n_kv_head;
     const int lane = threadIdx.x & 63, hg = threadIdx.x >> 6;
@@ -388,25 +390,41 @@ __global__ __launch_bounds__(512) void k_attn_scores(AttnArgs a) {
     if (start >= n) return;
     const int rows = (int)min((size_t)ATT_CH, n - start);
     const size_t kv = (size_t)a.n_kv_head * HD, q_dim = (size_t)a.n_head * HD;
-    for (int e = lane; e < HD; e += 64) sq[hg][e] = a.q[i * q_dim + (size_t)(kvh * gqa + hg) * HD + e];
     const float *kb = a.k_cache + start * kv + (size_t)kvh * HD;
     constexpr int R4 = HD / 4;
-    for (int idx = threadIdx.x; idx < rows * R4; idx += blockDim.x) {
-        const int r = idx / R4, c4 = idx % R4;
-        const float4 k4 = *(const float4 *)(kb + (size_t)r * kv + 4 * c4);
-        float *d = sk + r * KS + 4 * c4;
-        d[0] = k4.x;
-        d[1] = k4.y;
-        d[2] = k4.z;
-        d[3] = k4.w;
+    const int last = rows * R4 - 1, nth = (int)blockDim.x;
+    const float *qs = a.q + i * q_dim + (size_t)(kvh * gqa + hg) * HD;
+    float qv[HD / 64];
+#pragma unroll
+    for (int j = 0; j < HD / 64; j++) qv[j] = qs[lane + 64 * j];
+    for (int i0 = threadIdx.x; i0 <= last; i0 += 8 * nth) {
+        float4 k4[8];  // (past the end: the last piece again, stored where it is)
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int idx = min(i0 + j * nth, last);
+            k4[j] = *(const float4 *)(kb + (size_t)(idx / R4) * kv + 4 * (idx % R4));
+        }
+#pragma unroll
+        for (int j = 0; j < 8; j++) {
+            const int idx = min(i0 + j * nth, last);
+            *(float4 *)(sk + idx / R4 * KS + 4 * (idx % R4)) = k4[j];
+        }
     }
+#pragma unroll
+    for (int j = 0; j < HD / 64; j++) sq[hg][lane + 64 * j] = qv[j];
     __syncthreads();
     if (lane >= rows) return;
-    const float *kr = sk + lane * KS;
-    const float *qq = sq[hg];
+    const float4 *kr = (const float4 *)(sk + lane * KS);
+    const float4 *qq = (const float4 *)sq[hg];
     float s = 0.0f;
-#pragma unroll 16
-    for (int d = 0; d < HD; d++) s += qq[d] * kr[d];
+#pragma unroll 8
+    for (int d4 = 0; d4 < HD / 4; d4++) {
+        const float4 k4 = kr[d4], q4 = qq[d4];
+        s += q4.x * k4.x;
+        s += q4.y * k4.y;
+        s += q4.z * k4.z;
+        s += q4.w * k4.w;
+    }
     a.prob[(i * a.n_head + (size_t)(kvh * gqa + hg)) * a.span + (start + lane - t0)] = s * a.scale;
 }
 
