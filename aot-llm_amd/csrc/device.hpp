@@ -147,10 +147,25 @@ __device__ __forceinline__ bool exc_lookup(const uint32_t (*tab)[2], int n, uint
 // expf / tanhf bit-identical to the host libm the reference links against.
 // aotk_expf_tab reads the 2^(i/32) table from a copy (exp_table_to_lds: in
 // LDS a lookup costs an LDS read instead of a constant-memory load).
+// The few inputs where the restated algorithm differs are compared as
+// immediates, after the common path, and that path's ends are selects: a search
+// of the constant table (a divergent loop with a memory load in every call) and
+// the branches kept a thread's exps from overlapping. Prompt softmax of 64 rows
+// x 32 heads x 4032 positions 41.6 -> 32.8 us, the Llama-3-8B prompt of 512
+// tokens 46.5 -> 45.8 ms, a decode step behind it 2.29 -> 2.28 ms.
 __device__ __forceinline__ float aotk_expf_tab(float x, const uint64_t *tab) {
-    uint32_t o;
-    if (AOTK_EXPF_EXC_N && exc_lookup(expf_exc, AOTK_EXPF_EXC_N, __float_as_uint(x), o)) return __uint_as_float(o);
-    return lm_expf_tab(x, tab);
+    const uint32_t u = __float_as_uint(x);
+    if constexpr (AOTK_EXPF_EXC_N > 8) {
+        uint32_t o;
+        if (exc_lookup(expf_exc, AOTK_EXPF_EXC_N, u, o)) return __uint_as_float(o);
+        return lm_expf_tab(x, tab);
+    } else {
+        constexpr uint32_t exc[][2] = {AOTK_EXPF_EXC_DATA};
+        float f = lm_expf_tab(x, tab);
+#pragma unroll
+        for (int k = 0; k < AOTK_EXPF_EXC_N; k++) f = u == exc[k][0] ? __uint_as_float(exc[k][1]) : f;
+        return f;
+    }
 }
 __device__ __forceinline__ float aotk_expf(float x) { return aotk_expf_tab(x, lm_exp2f_tab_dev); }
 // The first 32 threads copy the table (the caller synchronises before use).

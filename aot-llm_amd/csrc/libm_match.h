@@ -90,13 +90,6 @@ LM_FN float lm_expf_tab(float x, const uint64_t *tab) {
     const double invln2n = 0x1.71547652b82fep+0 * 32;
     const double shift = 0x1.8p+52;
     const double c0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32, c1 = 0x1.ebfce50fac4f3p-3 / 32 / 32, c2 = 0x1.62e42ff0c52d6p-1 / 32;
-    uint32_t abstop = (lm_f2u(x) >> 20) & 0x7ff;
-    if (abstop >= ((lm_f2u(88.0f) >> 20) & 0x7ff)) {
-        if (lm_f2u(x) == lm_f2u(-INFINITY)) return 0.0f;
-        if (abstop >= ((lm_f2u(INFINITY) >> 20) & 0x7ff)) return x + x;
-        if (x > 0x1.62e42ep6f) return INFINITY;
-        if (x < -0x1.9fe368p6f) return 0.0f;
-    }
     double xd = (double)x;
     double z = invln2n * xd;
     double kd = z + shift;
@@ -111,7 +104,12 @@ LM_FN float lm_expf_tab(float x, const uint64_t *tab) {
     double y = lm_fma(c2, r, 1.0);
     y = lm_fma(zz, r2, y);
     y = y * s;
-    return (float)y;
+    /* the ends last, as selects: no branch, so that neighbouring calls
+     * interleave (the value computed above is unused there) */
+    float f = (float)y;
+    f = x > 0x1.62e42ep6f ? INFINITY : f;
+    f = x < -0x1.9fe368p6f ? 0.0f : f;
+    return x != x ? x + x : f;
 }
 
 LM_FN float lm_expf(float x) {
