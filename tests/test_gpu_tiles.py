@@ -185,3 +185,23 @@ def test_decode_attention_chunks(aotk, oracle, hd, span):
     vc[1::5] *= np.float32(1e-39)
     got = aotk.attention(q, kc, vc, 4, 2, hd, span, 0, span - 1, 1, 0)
     assert same_bits(got, attention_ref(oracle, q, kc, vc, 4, 2, hd, span, span - 1, 1, 0))
+
+
+def test_exp_at_its_ends(aotk, oracle):
+    """SiLU and softmax where exp leaves its common path: over- and underflow
+    and the values beside them, infinities, subnormal results and the inputs
+    that are compared one by one."""
+    ends = np.array([0x42b17217, 0x42b17218, 0x42b17219, 0x42b00000, 0xc2cff1b4, 0xc2cff1b5, 0xc2cff1b6, 0xc2aeac50, 0xc2b00000,
+                     0x4202422f, 0x4202422e, 0xc27c65d9, 0xc27c65da, 0x7f800000, 0xff800000, 0x7f7fffff, 0xff7fffff,
+                     0x00000001, 0x80000001], np.uint32).view(np.float32)
+    h = np.concatenate([ends, -ends])
+    up = np.ones_like(h)
+    ref = h.copy()
+    oracle.load().or_silu_mul(oracle.ptr(ref), oracle.ptr(up), ref.size)
+    got = aotk.silu_mul(h, up)
+    nan = np.isnan(ref)
+    assert np.array_equal(np.isnan(got), nan) and same_bits(got[~nan], ref[~nan])
+    s = np.concatenate([[0.0], np.minimum(ends, 0)]).astype(np.float32)
+    ref = s.copy()
+    oracle.load().or_softmax(oracle.ptr(ref), ref.size)
+    assert same_bits(aotk.softmax(s), ref)
