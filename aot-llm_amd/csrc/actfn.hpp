@@ -120,7 +120,7 @@ __device__ __forceinline__ void quant256(const float v[4], int lane, size_t blk,
         if (q80.xh) {  // batches: the tiled f16 copy; elements 4*lane .. +3 are one 8-byte run there
             const uint32_t h01 = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)qv[0]) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)qv[1]) << 16);
             const uint32_t h23 = (uint32_t)__builtin_bit_cast(uint16_t, (_Float16)qv[2]) | ((uint32_t)__builtin_bit_cast(uint16_t, (_Float16)qv[3]) << 16);
-            *(uint2 *)(q80.xh + q80_tiled_off(q80.tok, (int)blk * 8 + lane / 8, q80.nbt, 4 * (lane & 7))) = make_uint2(h01, h23);
+            *(uint2 *)(q80.xh + q80_tiled_off(q80.tok, (int)blk * 8 + lane / 8, q80.nbt, q80.xrows, 4 * (lane & 7))) = make_uint2(h01, h23);
         }
         if ((lane & 7) == 0) q80.d[blk * 8 + lane / 8] = d;
     }

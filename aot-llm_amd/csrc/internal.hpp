@@ -71,12 +71,14 @@ struct ActQ8_0 {
     int8_t *qs;     // [rows][n]
     float *d;       // [rows][n/32]
     // Batches of 2 or more: the quants as f16 in the matrix-core operand
-    // order (null = none), 1 KB per 16-vector tile and block of 32, tiles
-    // outer: [tile][block][group q < 4][vector v % 16][groups q, q + 4 of 4
-    // values] (see k_mm_q8).
+    // order (null = none), tiles of 16 vectors outer: [tile][block][group
+    // q < 4][vector of the tile][groups q, q + 4 of 4 values] (see k_mm_q8).
     uint16_t *xh;
-    int tok;  // vector index of this view's first row
-    int nbt;  // blocks of 32 per vector of the tiled copy
+    int tok;   // vector index of this view's first row
+    int nbt;   // blocks of 32 per vector of the tiled copy
+    int xrows; // vectors the tiled copy has places for: whole tiles, 1 KB per
+               // block, or, where memory is fixed and those do not fit, just
+               // the batch's, the last tile 64 bytes per vector and block
 };
 
 // Bytes of an activation buffer for `rows` vectors of n elements.
@@ -105,15 +107,21 @@ __host__ __device__ inline size_t q8k_tiled_off(size_t v, int sb, int nbt, int e
     const int j = e >> 5, g = (e >> 3) & 3;
     return ((v >> 4) * (size_t)nbt + sb) * 4096 + (size_t)((j >> 1) * 1024 + (g * 16 + (int)(v & 15)) * 16 + (j & 1) * 8 + (e & 7));
 }
+// Places in the 16-vector tile of vector v (ActQ8_0::xrows).
+__host__ __device__ inline int q80_tile_rows(size_t v, int xrows) {
+    const int left = xrows - (int)(v & ~(size_t)15);
+    return left < 16 ? left : 16;
+}
 // Value index in the tiled f16 copy of element e of block b of vector v.
-__host__ __device__ inline size_t q80_tiled_off(size_t v, int b, int nbt, int e) {
-    const int q = (e >> 2) & 3, half = e >> 4;
-    return ((v >> 4) * (size_t)nbt + b) * 512 + (size_t)((q * 16 + (int)(v & 15)) * 8 + half * 4 + (e & 3));
+__host__ __device__ inline size_t q80_tiled_off(size_t v, int b, int nbt, int xrows, int e) {
+    const int q = (e >> 2) & 3, half = e >> 4, tv = q80_tile_rows(v, xrows);
+    return (v >> 4) * (size_t)nbt * 512 + (size_t)b * (32 * tv) + (size_t)((q * tv + (int)(v & 15)) * 8 + half * 4 + (e & 3));
 }
-inline size_t act_q8_0_bytes(size_t n, size_t rows) {
-    return align_up(rows * n, 256) + align_up(rows * (n / 32) * 4, 256) +
-           (rows >= 2 ? align_up(align_up(rows, 16) * n * 2, 256) : 0);
+// xrows: the places of the tiled copy (whole tiles, or `rows`).
+inline size_t act_q8_0_bytes(size_t n, size_t rows, size_t xrows) {
+    return align_up(rows * n, 256) + align_up(rows * (n / 32) * 4, 256) + align_up(xrows * n * 2, 256);
 }
+inline size_t act_q8_0_bytes(size_t n, size_t rows) { return act_q8_0_bytes(n, rows, rows >= 2 ? align_up(rows, 16) : 0); }
 inline ActQ8_0 act_q8_0_view(void *base, size_t n, size_t rows) {
     uint8_t *p = (uint8_t *)base;
     ActQ8_0 a;
@@ -124,6 +132,7 @@ inline ActQ8_0 act_q8_0_view(void *base, size_t n, size_t rows) {
     a.xh = rows >= 2 ? (uint16_t *)p : nullptr;
     a.tok = 0;
     a.nbt = (int)(n / 32);
+    a.xrows = (int)align_up(rows, 16);
     return a;
 }
 

@@ -402,7 +402,7 @@ __global__ void k_quant_q8_0(const float *__restrict__ x, size_t nblk, ActQ8_0 o
     float id = d != 0.0f ? 1.0f / d : 0.0f;
     const int q = clampi(round_i(v * id), -127, 127);
     out.qs[i] = (int8_t)q;
-    if (out.xh) out.xh[q80_tiled_off(blk / out.nbt, (int)(blk % out.nbt), out.nbt, (int)(i & 31))] = __builtin_bit_cast(uint16_t, (_Float16)q);
+    if (out.xh) out.xh[q80_tiled_off(blk / out.nbt, (int)(blk % out.nbt), out.nbt, out.xrows, (int)(i & 31))] = __builtin_bit_cast(uint16_t, (_Float16)q);
     if ((i & 31) == 0) out.d[blk] = d;
 }
 
@@ -466,7 +466,7 @@ __global__ void k_ref_to_q8_0(const aotk_block_q8_0 *in, size_t nblk, ActQ8_0 a)
     size_t b = i / 32;
     int e = (int)(i % 32);
     a.qs[i] = in[b].qs[e];
-    if (a.xh) a.xh[q80_tiled_off(b / a.nbt, (int)(b % a.nbt), a.nbt, e)] = __builtin_bit_cast(uint16_t, (_Float16)in[b].qs[e]);
+    if (a.xh) a.xh[q80_tiled_off(b / a.nbt, (int)(b % a.nbt), a.nbt, a.xrows, e)] = __builtin_bit_cast(uint16_t, (_Float16)in[b].qs[e]);
     if (e == 0) a.d[b] = in[b].d;
 }
 

@@ -284,11 +284,10 @@ static int stage_act(const DevWeight &w, const void *x_dev, size_t m, ActQ8K &qk
     if (a == ACT_Q8_K || a == ACT_Q8_0) {
         const size_t need = a == ACT_Q8_K ? act_q8k_bytes(w.cols, m) : act_q8_0_bytes(w.cols, m);
         void *s;
-        // (the Q8_0 copy's whole 16-vector tiles are not counted against
-        // the fixed memory: where they do not fit, the copy is left out and
-        // the product runs without the matrix cores)
-        const size_t must = a == ACT_Q8_K ? need : align_up(m * w.cols, 256) + align_up(m * (w.cols / 32) * 4, 256) +
-                                                       align_up(m * w.cols * 2, 256);
+        // (the padding of the Q8_0 copy to whole 16-vector tiles is not
+        // counted against the fixed memory: where it does not fit, the last
+        // tile is laid out for the vectors it has)
+        const size_t must = a == ACT_Q8_K ? need : act_q8_0_bytes(w.cols, m, m);
         if (fixed) {
             if (must > fixed_cap)
                 return fail("matmul_noalloc: %zu inputs of %zu columns need %zu staging bytes, above the fixed %zu", m,
@@ -304,7 +303,7 @@ static int stage_act(const DevWeight &w, const void *x_dev, size_t m, ActQ8K &qk
             act = &qk;
         } else {
             q0 = act_q8_0_view(s, w.cols, m);
-            if (fixed && need > fixed_cap) q0.xh = nullptr;
+            if (fixed && need > fixed_cap) q0.xrows = (int)m;
             launch_ref_to_q8_0((const aotk_block_q8_0 *)x_dev, w.cols, m, q0, g_stream);
             act = &q0;
         }
