@@ -235,3 +235,81 @@ def test_exp_at_its_ends(aotk, oracle):
     ref = s.copy()
     oracle.load().or_softmax(oracle.ptr(ref), ref.size)
     assert same_bits(aotk.softmax(s), ref)
+
+
+def same_or_nan(got, ref):
+    """Equal bits, and NaN exactly where the reference has one (which NaN is
+    not part of the contract)."""
+    got, ref = np.asarray(got).reshape(-1), np.asarray(ref).reshape(-1)
+    nan = np.isnan(ref)
+    return np.array_equal(np.isnan(got), nan) and same_bits(got[~nan], ref[~nan])
+
+
+@pytest.mark.parametrize("kind", [F16, BF16, F32])
+@pytest.mark.parametrize("cols,m", [(136, 20), (256, 37)])
+def test_float_matmul_not_finite(aotk, oracle, kind, cols, m):
+    """Infinities and NaN in weights and inputs, in whole and partial stages,
+    and sums that overflow: the fused multiply-add's results, NaN payloads and
+    signs among them, and other rows and tokens keep their bits."""
+    rng = np.random.default_rng(cols + kind)
+    rows = 70
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    w[3, 0], w[17, cols - 1], w[40, 5], w[41, 9], w[64] = np.inf, np.nan, -np.inf, 60000.0, 0.0
+    w.view(np.uint32)[17, cols - 1] = 0xFFC12000  # payload bits that bf16 keeps
+    xs = rng.standard_normal((m, cols)).astype(np.float32)
+    xs[2, 7], xs[9, cols - 3], xs[15, 1], xs[11, ::2] = np.inf, np.nan, -np.inf, 3e38
+    xs.view(np.uint32)[9, cols - 3] = 0x7FC34567
+    raw = oracle.quantize_rows(kind, w)
+    h = aotk.Weight(kind, raw, rows, cols)
+    got = aotk.matmul(h, xs, m)
+    h.free()
+    ref = oracle.matmul(kind, raw, xs.view(np.uint8).reshape(-1), m, rows, cols, pool=oracle.Pool(8))
+    assert np.isnan(ref).any() and np.isinf(ref).any() and np.isfinite(ref).mean() > 0.5
+    assert same_bits(got.reshape(-1), ref.reshape(-1))
+
+
+@pytest.mark.parametrize("kind", [Q8_0, Q4_0, Q5_0])
+@pytest.mark.parametrize("cols,m", [(288, 13), (256, 20), (288, 37), (544, 64)])
+def test_q80_family_matmul_not_finite(aotk, oracle, kind, cols, m):
+    """Infinite and NaN block scales of weights and inputs (the last block's,
+    which the blocks past the end repeat, among them), scale products that
+    overflow, and an infinite scale times a zero quant."""
+    rng = np.random.default_rng(cols + kind + m)
+    rows, nb = 40, cols // 32
+    w = (rng.standard_normal((rows, cols)) * 0.02).astype(np.float32)
+    w[3, 0:4] = 0.0
+    raw = np.array(oracle.quantize_rows(kind, w)).view(np.uint8).reshape(rows, nb, -1)
+
+    def put(row, blk, v):
+        raw[row, blk, :2] = np.float16([v]).view(np.uint8)
+    put(3, 0, np.inf), put(17, nb - 1, np.nan), put(18, nb - 1, -np.inf), put(20, 2, 60000.0)
+    acts = np.stack([np.ascontiguousarray(oracle.quantize_act(kind, x.astype(np.float32))).view(np.uint8).reshape(nb, 36)
+                     for x in rng.standard_normal((m, cols))])
+    for tok, blk, v in ((2, 1, np.inf), (9, nb - 1, np.nan), (10, nb - 1, np.inf), (11, 2, 1e38)):
+        acts[tok, blk, :4] = np.float32([v]).view(np.uint8)
+    h = aotk.Weight(kind, raw.reshape(-1), rows, cols)
+    got = aotk.matmul(h, acts.reshape(-1), m)
+    h.free()
+    ref = oracle.matmul(kind, raw.reshape(-1), acts.reshape(-1), m, rows, cols, pool=oracle.Pool(8))
+    assert np.isnan(ref).any() and np.isinf(ref).any() and np.isfinite(ref).mean() > 0.5
+    assert same_or_nan(got, ref)
+
+
+@pytest.mark.parametrize("nh,nkv,hd,pos0,m,window", [
+    (4, 4, 64, 30, 3, 0), (32, 4, 64, 400, 64, 0), (32, 8, 128, 900, 40, 0), (8, 4, 64, 700, 4, 0), (8, 4, 64, 1500, 4, 0),
+    (8, 4, 64, 3000, 4, 0), (8, 2, 128, 200, 20, 64), (8, 4, 256, 90, 21, 0)])
+def test_prompt_attention_scores_not_finite(aotk, oracle, nh, nkv, hd, pos0, m, window):
+    """Infinite and NaN scores at positions that the rows hold: +inf and NaN
+    make a row NaN, -inf leaves the position out, and a kv head of nothing but
+    infinities is NaN."""
+    rng = np.random.default_rng(pos0 + m)
+    ctx = pos0 + m + 3
+    q = rng.standard_normal((m, nh, hd)).astype(np.float32)
+    kc, vc = (rng.standard_normal((ctx, nkv, hd)).astype(np.float32) for _ in range(2))
+    kc[pos0 - 3, 0, 0] = np.inf   # scores of either sign by q's
+    kc[pos0 + m - 2, 1, 1] = np.nan  # held by the last two rows
+    kc[:, nkv - 1, 2] = -np.inf
+    got = aotk.attention(q.reshape(-1), kc.reshape(-1), vc.reshape(-1), nh, nkv, hd, ctx, 0, pos0, m, window)
+    ref = attention_ref(oracle, q.reshape(-1), kc.reshape(-1), vc.reshape(-1), nh, nkv, hd, ctx, pos0, m, window)
+    assert np.isnan(ref).any() and (np.isfinite(ref.reshape(m, nh, hd)).all(2).any() or nkv == 1)
+    assert same_or_nan(got, ref)
