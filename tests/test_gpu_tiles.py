@@ -1,5 +1,6 @@
 """The batched kernels at the edges of their tiles, bit for bit against the
 CPU oracle (the reference's order of every f32 sum, so no tolerance)."""
+import ctypes
 import time
 
 import numpy as np
@@ -189,6 +190,40 @@ def test_matvec_output_over_its_input(aotk, oracle, kind):
     lib = aotk.runtime._lib()
     assert lib.aotk_matvec(w.h, buf.ptr, buf.ptr) == 0
     assert same_bits(buf.to_numpy(np.float32, rows), oracle.matvec(kind, raw, x, rows, cols))
+
+
+@pytest.mark.parametrize("kind", [Q4_K, Q8_0])
+@pytest.mark.parametrize("n,at", [(1, 0), (1, 256), (3, 0), (3, 1024)])
+def test_matvec_outputs_over_the_input_in_many_rounds(aotk, oracle, kind, n, at):
+    """40000 rows, 5000 blocks: more than are resident, so that later blocks
+    start after earlier ones have stored. The only or the last of three outputs
+    starts `at` bytes into the input."""
+    rng = np.random.default_rng(kind + at)
+    cols, rows = 4096, [8, 24, 40000][3 - n:]
+    bs, ts = (256, 144) if kind == Q4_K else (32, 34)
+    x = np.ascontiguousarray(oracle.quantize_act(kind, rng.standard_normal(cols).astype(np.float32))).view(np.uint8).reshape(-1)
+    assert at < x.size
+    raws = []
+    for r in rows:
+        raw = rng.integers(0, 256, (r * cols // bs, ts), dtype=np.uint8)
+        raw[:, :2] = np.float16([1e-3]).view(np.uint8)
+        if kind == Q4_K:
+            raw[:, 2:4] = np.float16([2e-3]).view(np.uint8)
+        raws.append(raw.reshape(-1))
+    ws = [aotk.Weight(kind, raw, r, cols) for raw, r in zip(raws, rows)]
+    buf = aotk.DeviceBuffer(4 * rows[-1] + at)
+    buf.upload(x)
+    outs = [aotk.DeviceBuffer(4 * r) for r in rows[:-1]]
+    ptrs = [o.ptr for o in outs] + [buf.ptr + at]
+    lib = aotk.runtime._lib()
+    if n == 1:
+        assert lib.aotk_matvec(ws[0].h, buf.ptr, ptrs[0]) == 0
+    else:
+        assert lib.aotk_matvec3((ctypes.c_void_p * 3)(*[w.h for w in ws]), buf.ptr, (ctypes.c_void_p * 3)(*ptrs)) == 0
+    got = [o.to_numpy(np.float32) for o in outs] + [buf.to_numpy(np.uint8)[at:].view(np.float32)]
+    for g, raw, r, w in zip(got, raws, rows, ws):
+        assert same_bits(g, oracle.matvec(kind, raw, x, r, cols))
+        w.free()
 
 
 @pytest.mark.parametrize("kind,rows,cols,m", [(Q4_K, 2048, 256, 2), (Q6_K, 2050, 768, 17), (Q5_K, 100, 2304, 33), (Q4_K, 33, 512, 16)])
