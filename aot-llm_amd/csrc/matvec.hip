@@ -1952,7 +1952,8 @@ __device__ __forceinline__ float hsum8(const float (&c)[8]) {
 
 // Q8_0 / Q4_0 / Q5_0 on the f16 matrix cores. The reference's integer part
 // per block is, for each of the 8 lanes of its accumulator, a sum of 4
-// consecutive products P_l (exact: |q| <= 127, |P_l| <= 64516).
+// consecutive products P_l (stored bytes may be -128 on both sides: |P_l| <=
+// 4 * 128 * 128 = 65536, exact).
 // v_mfma_f32_4x4x4_16b_f16 is sixteen independent 4x4 products of depth 4:
 // with A's blocks broadcast along the token axis (cbsz 2) and B's along the
 // row axis (blgp), one of them is P_l for 16 rows x 16 tokens, and eight take

@@ -330,6 +330,26 @@ def test_q80_family_matmul_not_finite(aotk, oracle, kind, cols, m):
     assert same_or_nan(got, ref)
 
 
+@pytest.mark.parametrize("m", [2, 20, 64])
+def test_q8_0_matmul_extreme_quants(aotk, m):
+    """Stored bytes of -128 on both sides, whole groups of them among others.
+    Scales of 1: every partial sum is an integer below 2^24, so the result is
+    the integers' own. (The reference's sign trick wraps on inputs of -128,
+    which its quantizer never makes.)"""
+    rng = np.random.default_rng(m)
+    rows, cols = 33, 288
+    w, x = (rng.integers(-128, 128, s, dtype=np.int8) for s in ((rows, cols), (m, cols)))
+    w[::3], x[1::2], w[1, ::2], x[0, :40] = -128, -128, 127, 127
+    raw = np.concatenate([np.full((rows, cols // 32, 1), 1, np.float16).view(np.uint8), w.view(np.uint8).reshape(rows, -1, 32)], 2)
+    acts = np.concatenate([np.full((m, cols // 32, 1), 1, np.float32).view(np.uint8), x.view(np.uint8).reshape(m, -1, 32)], 2)
+    h = aotk.Weight(Q8_0, raw.reshape(-1), rows, cols)
+    want = x.astype(np.int64) @ w.astype(np.int64).T
+    assert np.abs(want).max() == cols * 128 * 128
+    assert same_bits(aotk.matmul(h, acts.reshape(-1), m), want.astype(np.float32))
+    assert same_bits(aotk.matvec(h, acts[1].reshape(-1)), want[1].astype(np.float32))
+    h.free()
+
+
 @pytest.mark.parametrize("nh,nkv,hd,pos0,m,window", [
     (4, 4, 64, 30, 3, 0), (32, 4, 64, 400, 64, 0), (32, 8, 128, 900, 40, 0), (8, 4, 64, 700, 4, 0), (8, 4, 64, 1500, 4, 0),
     (8, 4, 64, 3000, 4, 0), (8, 2, 128, 200, 20, 64), (8, 4, 256, 90, 21, 0)])
