@@ -1917,15 +1917,11 @@ static bool mv_half_fits(const MvArgs &a) {
 // ------------------------------------------- prompt matmul: Q8_0 family, floats
 // Batches of 2 or more tokens for the kinds whose reference kernels keep 8
 // f32 lanes (dot_*_q8_0 / dot_f16_f32 ..., simd_avx2.rs:58-129, 433-493, and
-// their x4 forms, :273-330, bit-identical to the singles). Lane = token (64
-// per grid row), wave = MQ_R weight rows, block = 4 waves. A wave's weights
-// are the same for all its lanes: scalar loads (s_load), the nibble unpacking
-// on the scalar unit. The activation tile of a stage (MQ_BS blocks of 32, or
-// 64 float elements, for 64 tokens) is staged in LDS, two stages in turn,
-// with the next stage's loads in flight during the current one. Per
-// (row, token) the 8 chains run in element order exactly as in the matvec
-// kernels, then the avx2 horizontal sum (and, for floats, the scalar tail):
-// a batch equals m matvecs bit for bit.
+// their x4 forms, :273-330, bit-identical to the singles): k_mm_q8 on the f16
+// matrix cores, k_mm_fx on the f32 ones, k_mm_float on the VALU for rows that
+// are not whole 8-value groups. In each the 8 chains of a (row, token) run in
+// element order exactly as in the matvec kernels, then the avx2 horizontal sum
+// (and, in k_mm_float, the scalar tail): a batch equals m matvecs bit for bit.
 constexpr int MQ_R = 4;  // rows per wave of k_mm_float
 
 typedef uint32_t u32x4_t __attribute__((ext_vector_type(4)));
@@ -1936,13 +1932,6 @@ typedef uint32_t u32x8_t __attribute__((ext_vector_type(8)));
 template <typename T>
 __device__ __forceinline__ T uload(const void *p) {
     return *(const __attribute__((address_space(4))) T *)p;
-}
-
-// f16 element i of a uniform array of halves (4-byte aligned scalar load).
-__device__ __forceinline__ uint32_t uload_half(const uint16_t *base, size_t i) {
-    const uintptr_t at = (uintptr_t)(base + i);
-    const uint32_t v = uload<uint32_t>((const void *)(at & ~(uintptr_t)3));
-    return (at & 2) ? v >> 16 : v & 0xFFFFu;
 }
 
 __device__ __forceinline__ float hsum8(const float (&c)[8]) {
@@ -2414,8 +2403,11 @@ static void launch_mm_fx(const MvArgs &a, int m, hipStream_t s) {
 }
 
 // F16 / BF16 / F32 rows of other widths (4-byte aligned rows, a scalar tail;
-// whole 8-value groups take k_mm_fx): stage = 64 elements x 64 tokens of f32
-// input.
+// whole 8-value groups take k_mm_fx). Lane = token (64 per grid row), wave =
+// MQ_R weight rows, block = 4 waves. A wave's weights are the same for all its
+// lanes: scalar loads. The input is staged in LDS, 64 elements x 64 tokens of
+// f32, two stages in turn, with the next stage's loads in flight during the
+// current one.
 template <int KIND>
 __global__ __launch_bounds__(256) void k_mm_float(MvArgs a, int m) {
     __shared__ __align__(16) float sx[2][8][64][8];  // [stage][group of 8][token][element]
