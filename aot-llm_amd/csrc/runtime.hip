@@ -486,7 +486,7 @@ int aotk_attention(float *out_dev, const float *q_dev, const float *k_cache_dev,
                    size_t n_kv_head, size_t head_dim, size_t ctx, size_t layer, size_t pos0, size_t m, size_t window) {
     if (ensure_init()) return -1;
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return fail("attention: head_dim %zu unsupported", head_dim);
-    if (n_kv_head == 0 || n_head % n_kv_head || n_head / n_kv_head > 8) return fail("attention: bad head counts");
+    if (n_head == 0 || n_kv_head == 0 || n_head % n_kv_head || n_head / n_kv_head > 8) return fail("attention: bad head counts");
     if (pos0 + m > ctx) return fail("attention: positions exceed the context");
     if (ctx > 16384) return fail("attention: context %zu exceeds 16384 positions", ctx);
     size_t kv = n_kv_head * head_dim;
@@ -542,8 +542,8 @@ static const char *kind_ok_matrix(const aotk_tensor &t) {
 static int validate_spec(const aotk_model_spec *s, size_t blob_len) {
     const aotk_dims &d = s->dims;
     if (d.n_layer == 0 || !s->layers) return fail("spec: no layers");
-    if (d.n_kv_head == 0 || d.n_head % d.n_kv_head) return fail("spec: n_head %llu not a multiple of n_kv_head %llu",
-                                                                 (unsigned long long)d.n_head, (unsigned long long)d.n_kv_head);
+    if (d.n_head == 0 || d.n_kv_head == 0 || d.n_head % d.n_kv_head)
+        return fail("spec: n_head %llu not a multiple of n_kv_head %llu", (unsigned long long)d.n_head, (unsigned long long)d.n_kv_head);
     if (d.n_head / d.n_kv_head > 8) return fail("spec: gqa > 8 unsupported");
     if (d.head_dim != 64 && d.head_dim != 128 && d.head_dim != 256) return fail("spec: head_dim %llu unsupported", (unsigned long long)d.head_dim);
     if (d.head_dim == 256 && d.n_head / d.n_kv_head > 4) return fail("spec: head_dim 256 supports at most 4 query heads per kv head");

@@ -141,6 +141,14 @@ def test_prompt_attention_tiles(aotk, oracle, nh, nkv, hd, pos0, m, window):
     assert same_bits(got, attention_ref(oracle, q, kc, vc, nh, nkv, hd, ctx, pos0, m, window))
 
 
+@pytest.mark.parametrize("nh,nkv,m", [(0, 4, 2), (0, 4, 1), (4, 0, 2), (5, 2, 2), (18, 2, 2), (4, 2, 0)])
+def test_attention_refuses_bad_head_counts_and_no_rows(aotk, nh, nkv, m):
+    """No query head used to reach a division by the group size."""
+    z = np.zeros(64 * 64, np.float32)
+    with pytest.raises(aotk.abi.AotkError):
+        aotk.attention(z, z, z, nh, nkv, 64, 16, 0, 4, m, 0)
+
+
 @pytest.mark.parametrize("nh,nkv,hd,pos0,m,window", [(8, 4, 128, 200, 9, 0), (32, 8, 128, 70, 64, 40), (8, 4, 256, 90, 21, 32)])
 def test_prompt_attention_masks_positions(aotk, oracle, nh, nkv, hd, pos0, m, window):
     """Infinities and NaN in cache rows that a query row does not hold (later
