@@ -245,9 +245,13 @@ struct QkvPost {
     float eps;
 };
 void launch_qkv_post(const QkvPost &p, size_t m, size_t pos0, const int *pos_dev, hipStream_t s);
+// Positions an attention row may span (the softmax holds a row's scores in
+// registers and LDS): the entry points refuse longer contexts.
+constexpr size_t ATT_MAX_CTX = 16384;
+// m >= 1 rows from position pos0 on.
 void launch_attention(float *out, const float *q, const float *k_cache, const float *v_cache, size_t n_head,
                       size_t n_kv_head, size_t head_dim, size_t ctx_rows, size_t pos0, size_t m, size_t window,
-                      const int *pos_dev, float *scratch, size_t scratch_bytes, hipStream_t s);
+                      float *scratch, hipStream_t s);
 size_t attention_scratch_bytes(size_t n_head, size_t head_dim, size_t ctx, size_t m);
 // Decode step (one row at *pos_dev or pos0): the q/k/v epilogue of `p`
 // (bias, q/k norms, rope, KV store) fused into the scores, then softmax and

@@ -368,7 +368,7 @@ __device__ __forceinline__ void row_range(const AttnArgs &a, size_t i, size_t &t
     t0 = (a.window > 0 && pos + 1 > a.window) ? pos + 1 - a.window : 0;
 }
 
-// Scores: block = (kv head, chunk of ATT_CH positions, row), gqa * 64
+// Scores of one row: block = (kv head, chunk of ATT_CH positions), gqa * 64
 // threads. The chunk's K rows are staged in LDS (coalesced row loads, eight per
 // thread in flight; row stride HD + 4: 16-byte rows, the 16-byte reads of 16
 // rows hit all banks); thread (query head of the group, position) then runs its
@@ -383,17 +383,16 @@ __global__ __launch_bounds__(512) void k_attn_scores(AttnArgs a) {
     const int gqa = a.n_head / a.n_kv_head;
     const int lane = threadIdx.x & 63, hg = threadIdx.x >> 6;
     const int kvh = blockIdx.x, c = blockIdx.y;
-    const size_t i = blockIdx.z;
     size_t t0, n;
-    row_range(a, i, t0, n);
+    row_range(a, 0, t0, n);
     const size_t start = t0 + (size_t)c * ATT_CH;
     if (start >= n) return;
     const int rows = (int)min((size_t)ATT_CH, n - start);
-    const size_t kv = (size_t)a.n_kv_head * HD, q_dim = (size_t)a.n_head * HD;
+    const size_t kv = (size_t)a.n_kv_head * HD;
     const float *kb = a.k_cache + start * kv + (size_t)kvh * HD;
     constexpr int R4 = HD / 4;
     const int last = rows * R4 - 1, nth = (int)blockDim.x;
-    const float *qs = a.q + i * q_dim + (size_t)(kvh * gqa + hg) * HD;
+    const float *qs = a.q + (size_t)(kvh * gqa + hg) * HD;
     float qv[HD / 64];
 #pragma unroll
     for (int j = 0; j < HD / 64; j++) qv[j] = qs[lane + 64 * j];
@@ -425,7 +424,7 @@ __global__ __launch_bounds__(512) void k_attn_scores(AttnArgs a) {
         s += q4.z * k4.z;
         s += q4.w * k4.w;
     }
-    a.prob[(i * a.n_head + (size_t)(kvh * gqa + hg)) * a.span + (start + lane - t0)] = s * a.scale;
+    a.prob[(size_t)(kvh * gqa + hg) * a.span + (start + lane - t0)] = s * a.scale;
 }
 
 // Products of 16 steps for four rows at once: v_mfma_f32_4x4x1_f32 with a
@@ -711,8 +710,8 @@ __global__ __launch_bounds__(HD == 256 ? 64 * (QKD_MAX_GQA_256 + 1) : 576) void 
     QK_TS(3);
 }
 
-// Softmax and output per (row, head, group of SV_DB dims): block of SEQ_T
-// threads.
+// Softmax and output of one row per (head, group of SV_DB dims): block of
+// SEQ_T threads.
 //   softmax (ops.rs:98-112): max, glibc-matched exp, the sequential sum (one
 //   thread for short spans, the exact parallel replay for spans of
 //   SV_SEQ_MIN..SEQ_MAX_N), multiply by 1/sum; the blocks of one head repeat
@@ -730,7 +729,7 @@ __global__ __launch_bounds__(HD == 256 ? 64 * (QKD_MAX_GQA_256 + 1) : 576) void 
 #ifndef SV_TS
 #define SV_TS(c, i)
 #endif
-constexpr int ATT_MAX_SPAN = 16384;
+constexpr int ATT_MAX_SPAN = (int)ATT_MAX_CTX;
 constexpr int SV_DB = 16;         // dims per block
 constexpr int SV_CP = 384;        // positions per chunk
 constexpr int SV_RS = SV_CP + 4;  // floats per dim row of the product buffer
@@ -750,16 +749,15 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_sv(AttnArgs a) {
     float *prod = reinterpret_cast<float *>(ubuf);
     const int tid = threadIdx.x, lane = tid & 63;
     const int h = blockIdx.x / (HD / DB), d0 = (blockIdx.x % (HD / DB)) * DB;
-    const size_t i = blockIdx.y;
     const int gqa = a.n_head / a.n_kv_head;
     const int kvh = h / gqa;
     size_t t0, n;
-    row_range(a, i, t0, n);
+    row_range(a, 0, t0, n);
     const int cnt = (int)(n - t0);
     const bool exact = cnt >= SV_SEQ_MIN && cnt <= SEQ_MAX_N;
     const int C = seq_chunk(cnt);
     auto at = [&](int t) { return exact ? seq_idx(t, C) : t; };
-    const float *ps = a.prob + (i * a.n_head + h) * a.span;
+    const float *ps = a.prob + (size_t)h * a.span;
     const size_t kv = (size_t)a.n_kv_head * HD;
     const float *vb = a.v_cache + t0 * kv + (size_t)kvh * HD + d0;
     constexpr int R4 = DB / 4;
@@ -870,7 +868,7 @@ __global__ __launch_bounds__(SEQ_T) void k_attn_sv(AttnArgs a) {
         }
     }
     ATT_TS(4);
-    if (tid < DB) a.out[i * (size_t)a.n_head * HD + (size_t)h * HD + d0 + tid] = o;
+    if (tid < DB) a.out[(size_t)h * HD + d0 + tid] = o;
 }
 
 // Decode attention in one launch for spans of at most AD_MAX_SPAN positions (the
@@ -1282,8 +1280,8 @@ static void launch_rows(const AttnArgs &a, size_t head_dim, size_t m, size_t lon
 #undef OUTL
 }
 
-static void launch_sv(const AttnArgs &a, size_t head_dim, size_t m, hipStream_t s) {
-    dim3 g((unsigned)(a.n_head * (head_dim / SV_DB)), (unsigned)m);
+static void launch_sv(const AttnArgs &a, size_t head_dim, hipStream_t s) {
+    const unsigned g = (unsigned)(a.n_head * (head_dim / SV_DB));
     switch (head_dim) {
     case 64: k_attn_sv<64><<<g, SEQ_T, 0, s>>>(a); break;
     case 128: k_attn_sv<128><<<g, SEQ_T, 0, s>>>(a); break;
@@ -1318,14 +1316,10 @@ static AttnArgs attn_args(float *out, const float *q, const float *k_cache, cons
 
 void launch_attention(float *out, const float *q, const float *k_cache, const float *v_cache, size_t n_head,
                       size_t n_kv_head, size_t head_dim, size_t ctx_rows, size_t pos0, size_t m, size_t window,
-                      const int *pos_dev, float *scratch, size_t scratch_bytes, hipStream_t s) {
-    (void)scratch_bytes;
-    AttnArgs a = attn_args(out, q, k_cache, v_cache, n_head, n_kv_head, head_dim, ctx_rows, pos0, window, pos_dev,
+                      float *scratch, hipStream_t s) {
+    AttnArgs a = attn_args(out, q, k_cache, v_cache, n_head, n_kv_head, head_dim, ctx_rows, pos0, window, nullptr,
                            scratch);
-    size_t span = window > 0 && window < ctx_rows ? window : ctx_rows;
-    dim3 grid((unsigned)n_kv_head, (unsigned)((span + ATT_CH - 1) / ATT_CH), (unsigned)m);
-    const unsigned threads = (unsigned)(64 * (n_head / n_kv_head));
-    if (m > 1 && !pos_dev) {
+    if (m > 1) {
         // Eight rows per wave where that still leaves about four blocks per
         // CU, else four. 64 rows: 32 heads x 4032 positions, head_dim 128, 61
         // us with eight, 66 with four (100 before); 8 heads x 7000, head_dim
@@ -1347,19 +1341,19 @@ void launch_attention(float *out, const float *q, const float *k_cache, const fl
         else if (head_dim == 128) SCL(128);
         else SCL(256);
 #undef SCL
-    } else {
-        switch (head_dim) {
-        case 64: k_attn_scores<64><<<grid, threads, 0, s>>>(a); break;
-        case 128: k_attn_scores<128><<<grid, threads, 0, s>>>(a); break;
-        default: k_attn_scores<256><<<grid, threads, 0, s>>>(a); break;
-        }
+        // the longest row spans min(pos0 + m, window) positions
+        launch_rows(a, head_dim, m, window > 0 && window < pos0 + m ? window : pos0 + m, s);
+        return;
     }
-    // the longest row spans min(pos0 + m, window) positions
-    const size_t longest = window > 0 && window < pos0 + m ? window : pos0 + m;
-    if (m > 1 && !pos_dev && longest <= (size_t)ATT_MAX_SPAN)
-        launch_rows(a, head_dim, m, longest, s);
-    else
-        launch_sv(a, head_dim, m, s);
+    const size_t span = window > 0 && window < ctx_rows ? window : ctx_rows;
+    const dim3 grid((unsigned)n_kv_head, (unsigned)((span + ATT_CH - 1) / ATT_CH));
+    const unsigned threads = (unsigned)(64 * (n_head / n_kv_head));
+    switch (head_dim) {
+    case 64: k_attn_scores<64><<<grid, threads, 0, s>>>(a); break;
+    case 128: k_attn_scores<128><<<grid, threads, 0, s>>>(a); break;
+    default: k_attn_scores<256><<<grid, threads, 0, s>>>(a); break;
+    }
+    launch_sv(a, head_dim, s);
 }
 
 void launch_attention_decode(float *out, const QkvPost &p, size_t ctx_rows, size_t pos0, size_t window,
@@ -1383,7 +1377,7 @@ void launch_attention_decode(float *out, const QkvPost &p, size_t ctx_rows, size
     case 128: k_attn_qk_decode<128><<<grid, threads, 0, s>>>(a, p); break;
     default: k_attn_qk_decode<256><<<grid, threads, 0, s>>>(a, p); break;
     }
-    launch_sv(a, p.head_dim, 1, s);
+    launch_sv(a, p.head_dim, s);
 }
 
 // ------------------------------------------------------------ elementwise

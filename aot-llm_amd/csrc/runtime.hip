@@ -488,13 +488,14 @@ int aotk_attention(float *out_dev, const float *q_dev, const float *k_cache_dev,
     if (head_dim != 64 && head_dim != 128 && head_dim != 256) return fail("attention: head_dim %zu unsupported", head_dim);
     if (n_head == 0 || n_kv_head == 0 || n_head % n_kv_head || n_head / n_kv_head > 8) return fail("attention: bad head counts");
     if (pos0 + m > ctx) return fail("attention: positions exceed the context");
-    if (ctx > 16384) return fail("attention: context %zu exceeds 16384 positions", ctx);
+    if (ctx > ATT_MAX_CTX) return fail("attention: context %zu exceeds %zu positions", ctx, ATT_MAX_CTX);
+    if (m == 0) return fail("attention: no rows");
     size_t kv = n_kv_head * head_dim;
     size_t bytes = attention_scratch_bytes(n_head, head_dim, ctx, m);
     void *s = lib_scratch(bytes);
     if (!s) return -1;
     launch_attention(out_dev, q_dev, k_cache_dev + layer * ctx * kv, v_cache_dev + layer * ctx * kv, n_head, n_kv_head,
-                     head_dim, ctx, pos0, m, window, nullptr, (float *)s, bytes, g_stream);
+                     head_dim, ctx, pos0, m, window, (float *)s, g_stream);
     return finish_op();
 }
 
@@ -858,7 +859,6 @@ struct aotk_state {
     ActQ8_0 a0;
     float *cs, *cs_local;
     float *attn_ws;
-    size_t attn_ws_bytes;
     float *am_ws;
     uint32_t *ctl;     // [0] token, [1] pos, [2] argmax / sampled, [3] generated count, [4] sampler window count
     uint32_t *tokens;  // [max_batch]
@@ -924,8 +924,8 @@ aotk_state *aotk_state_new(aotk_model *m, size_t ctx, size_t max_batch) {
         fail("null model");
         return nullptr;
     }
-    if (ctx == 0 || ctx > 16384) {
-        fail("context %zu must be in 1..16384", ctx);
+    if (ctx == 0 || ctx > ATT_MAX_CTX) {
+        fail("context %zu must be in 1..%zu", ctx, ATT_MAX_CTX);
         return nullptr;
     }
     if (max_batch < 1) max_batch = 1;
@@ -969,8 +969,7 @@ aotk_state *aotk_state_new(aotk_model *m, size_t ctx, size_t max_batch) {
         st->ak = act_q8k_view(ak, nmax, B);
         st->a0 = act_q8_0_view(a0, nmax, B);
     }
-    st->attn_ws_bytes = attention_scratch_bytes(d.n_head, d.head_dim, ctx, B);
-    st->attn_ws = (float *)alloc(st->attn_ws_bytes);
+    st->attn_ws = (float *)alloc(attention_scratch_bytes(d.n_head, d.head_dim, ctx, B));
     st->am_ws = F(1024);
     st->ctl = (uint32_t *)alloc(64);
     st->tokens = (uint32_t *)alloc(B * 4);
@@ -1084,7 +1083,7 @@ static void run_layers(aotk_state *st, size_t m, size_t pos0, const int *pos_dev
         } else {
             launch_qkv_post(p, m, pos0, pos_dev, s);
             launch_attention(st->xb, st->q, kc, vc, d.n_head, d.n_kv_head, d.head_dim, st->ctx, pos0, m, window,
-                             pos_dev, st->attn_ws, st->attn_ws_bytes, s);
+                             st->attn_ws, s);
         }
         // decode: the attention output is quantized inside the wo launch where the kind allows
         float *wo_y = f.post_norms ? st->xb2 : st->x;

@@ -130,10 +130,10 @@ def attention_ref(oracle, q, kc, vc, nh, nkv, hd, ctx, pos0, m, window):
     (32, 4, 64, 1984, 64, 0), (32, 4, 64, 1985, 64, 0), (32, 4, 64, 4032, 64, 0), (32, 4, 64, 4033, 64, 0),
     (32, 4, 64, 8128, 64, 0), (32, 4, 64, 8129, 64, 0),
     (8, 4, 64, 508, 4, 0), (8, 4, 64, 509, 4, 0), (8, 4, 64, 1020, 4, 0), (8, 4, 64, 1021, 4, 0),
-    (8, 4, 64, 2044, 4, 0), (8, 4, 64, 2045, 4, 0), (8, 4, 64, 8188, 4, 0), (8, 4, 64, 8189, 4, 0)])
+    (8, 4, 64, 2044, 4, 0), (8, 4, 64, 2045, 4, 0), (8, 4, 64, 8188, 4, 0), (8, 4, 64, 8189, 4, 0), (4, 2, 64, 16379, 2, 0)])
 def test_prompt_attention_tiles(aotk, oracle, nh, nkv, hd, pos0, m, window):
     rng = np.random.default_rng(nh * 7 + hd + pos0 + m)
-    ctx = pos0 + m + 3
+    ctx = pos0 + m + 3  # (at most the longest context, 16384)
     q = (rng.standard_normal(m * nh * hd) * 2).astype(np.float32)
     kc, vc = (rng.standard_normal(ctx * nkv * hd).astype(np.float32) for _ in range(2))
     vc[::5] *= np.float32(1e-39)  # products in the subnormals
@@ -141,12 +141,13 @@ def test_prompt_attention_tiles(aotk, oracle, nh, nkv, hd, pos0, m, window):
     assert same_bits(got, attention_ref(oracle, q, kc, vc, nh, nkv, hd, ctx, pos0, m, window))
 
 
-@pytest.mark.parametrize("nh,nkv,m", [(0, 4, 2), (0, 4, 1), (4, 0, 2), (5, 2, 2), (18, 2, 2), (4, 2, 0)])
-def test_attention_refuses_bad_head_counts_and_no_rows(aotk, nh, nkv, m):
+@pytest.mark.parametrize("nh,nkv,ctx,m", [(0, 4, 16, 2), (0, 4, 16, 1), (4, 0, 16, 2), (5, 2, 16, 2), (18, 2, 16, 2), (4, 2, 16, 0),
+                                          (4, 2, 16385, 1), (4, 2, 16385, 2)])
+def test_attention_refuses_bad_head_counts_no_rows_and_long_contexts(aotk, nh, nkv, ctx, m):
     """No query head used to reach a division by the group size."""
     z = np.zeros(64 * 64, np.float32)
-    with pytest.raises(aotk.abi.AotkError):
-        aotk.attention(z, z, z, nh, nkv, 64, 16, 0, 4, m, 0)
+    with pytest.raises(aotk.abi.AotkError, match="attention: "):
+        aotk.attention(z, z, z, nh, nkv, 64, ctx, 0, 4, m, 0)
 
 
 @pytest.mark.parametrize("nh,nkv,hd,pos0,m,window", [(8, 4, 128, 200, 9, 0), (32, 8, 128, 70, 64, 40), (8, 4, 256, 90, 21, 32)])
@@ -247,7 +248,7 @@ def test_kquant_staging_tiles(aotk, oracle, kind, rows, cols, m):
 
 
 @pytest.mark.parametrize("hd", [64, 128, 256])
-@pytest.mark.parametrize("span", [1, 64, 65, 320, 321, 384, 385, 448, 768, 769, 1023, 1152, 1537, 4609])
+@pytest.mark.parametrize("span", [1, 64, 65, 320, 321, 384, 385, 448, 768, 769, 1023, 1152, 1537, 4609, 16384])
 def test_decode_attention_chunks(aotk, oracle, hd, span):
     """One row over spans around the 64-value runs and the 384-position chunks
     of its ordered sums, signed zeros and subnormal products among them."""
