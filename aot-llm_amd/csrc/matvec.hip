@@ -1959,8 +1959,8 @@ __device__ __forceinline__ float hsum8(const float (&c)[8]) {
 // Bound by issue: per tile and block 64 + 8 clocks of matrix products and 32
 // fma of 2.4, which barely overlap. Q8_0 at 64 tokens, against 16x16x32
 // products with the groups laid out diagonally (7 of 8 factors zero) and the
-// activations staged in LDS: 12288x4096 82 -> 50 us, 4096x12288 114 -> 62,
-// 24576x4096 120 -> 96; 5632x2048 at 6 tokens 30 -> 14 (Q5_0 32 -> 16).
+// activations staged in LDS: 12288x4096 77 -> 46 us, 4096x12288 115 -> 61,
+// 24576x4096 122 -> 85; 5632x2048 at 6 tokens 27 -> 13.5 (Q5_0 30 -> 15.5).
 // Wave = one 16-token tile x CH of the 8 chains; block = 16 rows x 16 NT
 // tokens. The weights are converted to f16 into LDS once per block, 8 blocks
 // of 32 per stage; the activations come straight from the operand-ordered
@@ -2204,13 +2204,17 @@ static void launch_mm_q8(const MvArgs &a, int m, hipStream_t s) {
     const int gy = (tiles + 3) / 4, nt = (tiles + gy - 1) / gy;
     const dim3 grid(gx, (unsigned)gy);
     // A tile's chains on two waves for at most 32 tokens a block, where the
-    // SIMDs would otherwise hold too few waves (Q8_0, 16 tokens: 4096x4096 20
-    // against 26 us, 12288x4096 31 against 35, 4096x12288 59 against 73); on
-    // one wave above (64 tokens: 24 against 26, 50 against 76, 62 against 77:
-    // two waves form every scale product and read every operand line twice).
+    // SIMDs would otherwise hold too few waves (Q8_0, 16 tokens: 4096x4096 20.6
+    // against 23.6 us, 12288x4096 27.2 against 27.8, 4096x12288 53 against 61;
+    // 32 tokens: 4096x4096 21.2 / 22.5); on one wave above (64 tokens: 22.8
+    // against 26.6, 46 against 66, 61 against 69: two waves form every scale
+    // product and read every operand line twice). Tall matrices do not lack
+    // waves and are past the line at 17..32 tokens already, which the rule does
+    // not see: 12288x4096 at 32 tokens 38 with two, 33 with one, 24576x4096 68 /
+    // 48.
     const bool split = nt <= 2;
     // (a compile-time step between blocks where the tiles are whole: Q5_0
-    // 5632x2048 at 6 tokens 16.1 against 16.9 us)
+    // 5632x2048 at 6 tokens 16.1 against 16.9 us, the same run)
 #define Q8L(C, N)                                                                        \
     do {                                                                                 \
         if (a.xrows % 16 == 0) k_mm_q8<KIND, C, N, true><<<grid, 64 * N * (8 / C), 0, s>>>(a, m); \
@@ -2228,11 +2232,11 @@ static void launch_mm_q8(const MvArgs &a, int m, hipStream_t s) {
 
 // F16 / BF16 / F32 rows of whole 8-value groups on the f32 matrix cores.
 // v_mfma_f32_16x16x4_f32 is four fused multiply-adds in k order, each rounded
-// once (equal to fmaf bit for bit, denormals and infinities included), so it
-// runs four steps of one of the reference's 8 chains for 16 rows x 16 tokens:
-// chain l takes the values 8g + l of groups g = 4s..4s+3, and lane
-// (k = lane / 16, i = lane % 16) holds group 4s + k of row / token i, which is
-// 16 (F32: 32) consecutive bytes of a weight row and 32 of an input. Eight of
+// once (equal to fmaf bit for bit, denormals, infinities and NaN payloads
+// included), so it runs four steps of one of the reference's 8 chains for 16
+// rows x 16 tokens: chain l takes the values 8g + l of groups g = 4s..4s+3, and
+// lane (k = lane / 16, i = lane % 16) holds group 4s + k of row / token i, which
+// is 16 (F32: 32) consecutive bytes of a weight row and 32 of an input. Eight of
 // these, one per chain, take a 16x16 tile four groups on.
 // Block = 4 waves = 64 rows x 16 TT tokens, wave = 16 rows. A stage is 16
 // groups: whole-line global loads two stages ahead in registers, then LDS, two
@@ -2243,9 +2247,9 @@ static void launch_mm_q8(const MvArgs &a, int m, hipStream_t s) {
 // Groups past the last enter as 0 and -0, whose product leaves any
 // accumulator as it is.
 // Bound by the matrix cores: a tile step is 8 x 32 clocks and a lone wave per
-// SIMD spends about 60% of its time in them. F16 4096x4096: 37 tokens 147 ->
-// 30 us, 2 tokens 234 -> 29; 14336x4096 at 64 tokens 269 -> 91 us; F32
-// 4096x4096 266 -> 38 us (against the VALU kernel below).
+// SIMD spends about 60% of its time in them. F16 4096x4096: 37 tokens 127 ->
+// 29 us, 2 tokens 123 -> 29 (BF16 223 -> 30); 14336x4096 at 64 tokens 232 -> 90
+// us; F32 4096x4096 185 -> 36 us (against the VALU kernel below).
 typedef float f4u_t __attribute__((ext_vector_type(4), aligned(4)));
 typedef uint32_t u4u_t __attribute__((ext_vector_type(4), aligned(4)));
 constexpr int FX_STEP = 1024 + 64;  // bytes of 64 slots, padded: the steps of a row start 16 banks apart
@@ -2393,7 +2397,7 @@ __global__ __launch_bounds__(256) void k_mm_fx(MvArgs a, int m) {
 
 // Two token tiles per block where that takes no more rounds of blocks over
 // the 256 CUs (fewer readers of each weight), else one. F16 14336x4096 at 64
-// tokens: 91 us with two, 99 with one; 4096x4096: 49 with two, 30 with one.
+// tokens: 90 us with two, 97 with one; 4096x4096: 48 with two, 30 with one.
 template <int KIND>
 static void launch_mm_fx(const MvArgs &a, int m, hipStream_t s) {
     const unsigned gx = (unsigned)((a.total_rows + 63) / 64), tiles = (unsigned)((m + 15) / 16);

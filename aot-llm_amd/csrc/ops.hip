@@ -1236,24 +1236,35 @@ static void launch_rows(const AttnArgs &a, size_t head_dim, size_t m, size_t lon
     const unsigned pairs = (unsigned)(m * a.n_head);
 #define SML(P, CAP, T) k_attn_softmax_rows_p<P, CAP, T><<<(pairs + P - 1) / P, T, 0, s>>>(a, (int)m)
     if (pairs >= 1024 && longest <= 8192) {
-        // enough pairs for eight per block on every CU. 64 rows x 32 heads
-        // against one pair per wave, and past 1024 positions per 256 threads
-        // with the parallel replay: 512 positions 9.5 -> 7.3 us, 4096 50 ->
-        // 41 (33 since expf has no branches); 6064 (four per block) 95 -> 78
+        // enough pairs for eight per block on every CU (four past 4096
+        // positions: LDS). 64 rows x 32 heads, against one pair per wave and,
+        // past 1024 positions, 256 threads with the parallel replay: 500
+        // positions 10.0 -> 6.2 us, 1000 16.5 -> 9.9, 2000 31 -> 16.5, 4090 49
+        // -> 31, 6064 95 -> 65, 8100 112 -> 83. Against the replay of _x there:
+        // 34, 38, 45, 54, 66, 75; at 1024 pairs 2000 positions 15.6 / 23.5 us,
+        // 4090 27.8 / 28.5, 8100 44 / 41; at 768 pairs 3000 21.3 / 20.0, 4090
+        // 27.2 / 22.0. The next larger instance costs 0.1..0.9 us: 500
+        // positions 6.3, 1000 10.2, 2000 16.7.
         if (longest <= 512) SML(8, 512, 1024);
         else if (longest <= 1024) SML(8, 1024, 1024);
         else if (longest <= 2048) SML(8, 2048, 1024);
         else if (longest <= 4096) SML(8, 4096, 1024);
         else SML(4, 8192, 1024);
     } else if (longest <= 2048) {
-        // few pairs: more threads each (50 rows x 8 heads, a 1024 window
-        // 17.4 -> 8.0 us, 6.9 since expf has no branches; 6 rows x 32 heads, 2006 positions 35 -> 12.6)
+        // few pairs: more threads each. Against one pair per wave before: 50
+        // rows x 8 heads, a 1024 window 17.7 -> 6.5 us; 6 rows x 32 heads, 2006
+        // positions 34 -> 11.4. Against eight per block, 512 pairs: 500
+        // positions 5.6 / 6.0, 1000 7.4 / 9.2, 2000 12.0 / 15.6. (Measured, not
+        // used: at 64..256 pairs the replay is ahead from 1000 positions on,
+        // 2000 in 7.2 us; at 768 pairs eight per block from 1500, 2000 in 15.7
+        // against 19.3.)
         if (longest <= 512) SML(4, 512, 512);
         else if (longest <= 1024) SML(2, 1024, 512);
         else SML(2, 2048, 1024);
     } else if (longest <= 8192) {
         // few long rows: the parallel replay (20 rows x 8 heads, 3020
-        // positions: 8.2 us against 15 for one chain per block)
+        // positions: 7.0 us against 18 for four per block; 512 pairs, 4090
+        // positions 15.5 / 23)
         k_attn_softmax_rows_x<8192><<<pairs, SEQ_T, 0, s>>>(a, (int)m);
     } else {
         k_attn_softmax_rows_x<ATT_MAX_SPAN><<<pairs, SEQ_T, 0, s>>>(a, (int)m);
@@ -1261,10 +1272,10 @@ static void launch_rows(const AttnArgs &a, size_t head_dim, size_t m, size_t lon
 #undef SML
     // Items per wave: as many waves as there are SIMDs first, then more items
     // per product (each product instruction serves up to four). 64 rows x 32
-    // heads x 4032 positions (4096 / NI waves): NI 4 82 us, 2 118, 1 204
-    // (114 before, with V per wave from L2 and p from LDS); 64 rows x 8 heads
-    // x 7000, head_dim 256: NI 2 117, 4 132, 1 173 (156); 6 rows x 32 heads x
-    // 2000: NI 1 26, 2 33, 4 37 (41).
+    // heads x 4032 positions (4096 / NI waves): NI 4 79..88 us over a run, 2
+    // 115, 1 205 (117 before, with V per wave from L2 and p from LDS); 64 rows
+    // x 8 heads x 7000, head_dim 256: NI 2 118, 4 133, 1 176 (159); 6 rows x 32
+    // heads x 2000: NI 1 29, 2 35, 4 41 (45).
     const size_t items = m * (a.n_head / a.n_kv_head), per = a.n_kv_head * (head_dim / 64);
     const int NI = items * per <= 1024 ? 1 : items * per <= 2048 ? 2 : 4;
     const unsigned g = (unsigned)(per * ((items + 4 * NI - 1) / (4 * NI)));
@@ -1321,11 +1332,11 @@ void launch_attention(float *out, const float *q, const float *k_cache, const fl
                            scratch);
     if (m > 1) {
         // Eight rows per wave where that still leaves about four blocks per
-        // CU, else four. 64 rows: 32 heads x 4032 positions, head_dim 128, 61
-        // us with eight, 66 with four (100 before); 8 heads x 7000, head_dim
-        // 256, 59 / 66 (146); 32 heads x 448 14.5 / 13.9 (18); 8 heads, a
-        // 1024 window, head_dim 256, 20.7 / 19.5 (37); 6 rows x 32 heads x
-        // 2000 10.5 / 8.7 (11.4).
+        // CU, else four. 64 rows: 32 heads x 4032 positions, head_dim 128,
+        // 59..66 us over a run with eight, 69 with four (102 before); 8 heads x
+        // 7000, head_dim 256, 57 / 64 (147); 32 heads x 448 14.7 / 14.2 (17.6);
+        // 8 heads, a 1024 window, head_dim 256, 21.4 / 20.1 (40); 6 rows x 32
+        // heads x 2000 9.6 / 8.5 (10.6).
         const size_t held = window > 0 && window < pos0 + m ? window + m : pos0 + m;  // positions of any row
         const int gqa = (int)(n_head / n_kv_head), rgs = std::max(1, 4 / gqa);
         const size_t blocks8 = n_kv_head * ((held + ATT_CH - 1) / ATT_CH) * ((m + 8 * rgs - 1) / (8 * rgs));
