@@ -21,7 +21,7 @@ FLAGS = [
     "-O3", "-std=c++17", "-fPIC", "--offload-arch=gfx950",
     # bit-exactness: no implicit FMA contraction, IEEE division and sqrt
     "-ffp-contract=off", "-fhip-fp32-correctly-rounded-divide-sqrt",
-    # never emit packed-FP32 VALU ops (they are avoided on this pool)
+    # never emit packed-FP32 VALU ops (some of their forms have given wrong results)
     "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
     # matrix-core results in VGPRs (the f32 folds read them directly; the
     # AGPR form costs one v_accvgpr_read per value)
